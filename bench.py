@@ -9,7 +9,7 @@ passes timed with HIP events on the engine's stream.  Prints one JSON line.
 
   value         pair interactions evaluated per second (pairs per pass /
                 mean pass time)
-  roofline      the pair kernel (k_nonbond): 46 algorithmic FP32 FLOP per
+  roofline      the pair kernel (k_pair): 46 algorithmic FP32 FLOP per
                 evaluated pair over its mean launch time, against the FP32
                 peak; traffic from the committed rocprofv3 counter summary
   cpu_baseline  the FP64 oracle (CPU restatement of the reference runner)
@@ -49,7 +49,7 @@ FP32_PEAK_TFLOPS = 157.3    # MI355X FP32 peak
 # inputs runs each product twice; that precision work is not counted)
 MLP_MFMA_FLOP = 2 * 2 * 64 * 64
 BF16_PEAK_TFLOPS = 2500.0   # MI355X dense bf16 MFMA peak
-MI355X_CUS = 256            # the pair kernel's 5-wave build runs from 64 cells per CU up
+MI355X_CUS = 256
 DT_PS = 0.002               # 2 fs time step for ns/day
 MLP_TRAIN_STEPS = 40000     # surrogate training steps on the mixture (16,384 samples each)
 METRIC = "pair-interactions/s & ns/day at 1M atoms; MLP vs table at fixed force RMSE"
@@ -722,18 +722,12 @@ def eng_cells(sysm):
 def pair_kernel_name(sysm, md):
     """The pair kernel each upload picks: the half shell (with k_fold) for
     engine_gpu_half_mean or more atoms per cell on average in fewer cells
-    than the device has CUs, otherwise the full shell with paired visits,
-    followed by k_fold when the owners are split (that occupancy in fewer
-    than 32 cells per CU); the 5-wave build from 64 cells per CU."""
+    than the device has CUs, otherwise the full shell's k_pair, followed by
+    k_fold when the owners are split (12 work items per CU or fewer)."""
     cells = eng_cells(sysm)
-    wide = cells >= 64 * MI355X_CUS
-    dense = sysm.N >= md.engine_gpu_half_mean * cells
-    if dense and cells < MI355X_CUS:
-        return ("k_nonbond_half_wide" if wide else "k_nonbond_half") + " + k_fold"
-    name = "k_nonbond_paired_wide" if wide else "k_nonbond_paired"
-    if dense and cells < 32 * MI355X_CUS:
-        name += " + k_fold"
-    return name
+    if sysm.N >= md.engine_gpu_half_mean * cells and cells < MI355X_CUS:
+        return "k_nonbond_half + k_fold"
+    return "k_pair + k_fold" if 2 * cells <= 12 * MI355X_CUS else "k_pair"
 
 
 if __name__ == "__main__":

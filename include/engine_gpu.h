@@ -113,34 +113,32 @@ int engine_gpu_steps(struct engine *e, int nsteps, double *epot, double *ekin);
 #define engine_flag_mlp 131072
 /* Pair-kernel shell, chosen at every particle upload (each pass, each
    engine_gpu_steps call; no reference counterpart):
-   full shell    every pair evaluated by both of its atoms' cells, forces
-                 kept in registers;
+   full shell    every pair evaluated by both of its atoms' cells, no
+                 scattered forces;
    half shell    every pair task visited once, the opposite forces added in
                  LDS per visit and folded per atom in a fixed order.
    Without either flag the half shell is taken when the cells hold
    engine_gpu_half_mean atoms or more on average and are fewer than the
-   device's compute units (or engine_flag_unpaired is set): it saves work
-   there.  Otherwise the paired full shell is faster (100k water, 1000 cells
-   of 100 atoms: 0.69 against 0.75 ms), and with few atoms per cell the half
-   shell's per-visit cost outweighs its halved pair work.
+   device's compute units (or engine_flag_unpaired is set).  Otherwise the
+   full shell is taken: the half shell's opposite forces, LDS atomics, cost
+   more than the evaluations they save.
    The surrogate pass (engine_flag_mlp) takes the half shell unless
    engine_flag_fullshell is set: its network evaluation dominates a visit. */
 #define engine_flag_fullshell 262144
 #define engine_flag_halfshell 524288
 #define engine_gpu_half_mean 48
-/* Owner split (no reference counterpart): with fewer than 32 cells per
-   compute unit and engine_gpu_half_mean or more atoms per cell on average,
-   engine_gpu_load splits each owner cell's neighbour list into up to 8
-   groups, each a work item of the pair kernel with its own partial forces
-   and sums, folded per atom in group order.  engine_flag_nosplit keeps one
-   item per cell. */
+/* Owner split (no reference counterpart): with few cells engine_gpu_load
+   splits each owner cell's neighbour list into groups, each a work item of
+   the pair kernel with its own partial forces and sums, folded per atom in
+   group order: table pass, up to 32 groups and 12 items per compute unit;
+   half shell and surrogate, up to 8 groups below 32 cells per compute unit with
+   engine_gpu_half_mean or more atoms per cell on average.
+   engine_flag_nosplit keeps one item per cell. */
 #define engine_flag_nosplit 1048576
-/* Paired visits (no reference counterpart): the full-shell table kernel
-   visits the neighbour cells at opposite offsets +d and -d of an owner cell
-   together, so that each lane walks its atom's window into both (long on one
-   side where it is short on the other); with the reference window only
-   (engine_flag_projwindow passes visit one neighbour at a time).
-   engine_flag_unpaired visits them one at a time. */
+/* Unpaired visits (no reference counterpart): densely filled cells
+   (engine_gpu_half_mean) take the half shell however many they are, unless
+   engine_flag_fullshell is set.  No other effect: the table kernel takes a
+   cell's neighbours 64 at a time. */
 #define engine_flag_unpaired 2097152
 
 /* Species pairs: ti[p], tj[p] (ti <= tj) for p < returned count. */

@@ -15,38 +15,37 @@
  *               particles get a wave per direction and a wave-parallel
  *               restatement of that quicksort (sort_desc_wave); smaller
  *               cells one wave that sorts all their lists (sort_lists_wave);
- *   k_nonbond   persistent kernel: each wave pulls an owner cell from one of
- *               8 device queues (one per XCD slab of cells), walks the cell's
- *               neighbour list (the reference's self/pair tasks that touch
- *               it) and accumulates the forces of its own atoms only, so no
- *               atomics on forces and no cross-wave write conflicts.  Lanes
- *               are (owner atom, partition); per neighbour cell the positions
- *               and sorted words are prefetched one neighbour ahead and the
- *               cell is staged in LDS in window order as packed records
- *               (x, y, z, key | index << 16 | type << tshift).  Each lane walks
- *               its share of the sorted window (runner_dopair.c:455-478),
- *               keeps every record with r^2 up to the top of a thin band
- *               around rc^2 in a lane-private LDS list, then evaluates them
- *               two at a time, the band's pairs decided in FP64 first: FP32 table evaluation
- *               (potential_eval.h:67-104), forces summed in registers and
- *               folded into two-sum (hi, lo) accumulators per neighbour.
+ *   k_pair      (pair_tile.h) full shell, table mode: one wave per work item,
+ *               an owner cell and a share of its neighbour list (the
+ *               reference's self/pair tasks that touch it): matrix-core
+ *               distance filter, the hits dealt over the lanes, FP32 table
+ *               evaluation (potential_eval.h:67-104).  It accumulates the
+ *               forces of its own atoms only (every pair at both its cells),
+ *               so no atomics on forces and no cross-wave write conflicts.
  *               Excluded pairs are subtracted afterwards as in
- *               exclusion.c:81-282.  The queues hand out work items: owner
- *               cells in 6x6x6 blocks, each split over up to 8 neighbour
- *               groups when there are few, densely filled cells;
- *   k_nonbond_half (and the surrogate k_nonbond_mlp_half): each pair task
- *               is visited once, at its i cell; the opposite forces go into
- *               LDS copies of the visited cell and out to a per-visit slot;
+ *               exclusion.c:81-282;
+ *   k_nonbond_half
+ *               half shell, table mode: persistent waves pull owner cells from
+ *               8 device queues (one per XCD slab of cells) and visit each
+ *               pair task once, at its i cell.  Lanes are (owner atom,
+ *               partition); each neighbour cell is staged in LDS in window
+ *               order, each lane walks its share of the sorted window
+ *               (runner_dopair.c:455-478) and evaluates its hits; the opposite
+ *               forces go into LDS copies of the visited cell and out to a
+ *               slot per visit;
+ *   k_nonbond_mlp, k_nonbond_mlp_half
+ *               the surrogate's pass, full or half shell: the same walk, the
+ *               hits evaluated with the network;
  *   k_fold      per atom, the groups' partial forces and the half-shell
  *               slots, added in a fixed order;
  *   k_reduce_a/b per-item FP64 energies/virials/counts -> totals, fixed order.
  * Staged neighbour records hold their positions moved into the owner's
  * frame (x + shift, once per record), so a candidate's distance is one
- * subtraction per axis.  In the full-shell kernels every pair is evaluated
- * by both of its cells (once per owner); the two owners' FP32 distances are
- * opposite to rounding (each side rounds its own shifted position), so the
- * forces sum to zero to FP32 rounding; energy, virial and counts are taken
- * on the task's i side only.
+ * subtraction per axis.  In the full shell every pair is evaluated by both
+ * of its cells (once per owner); the two owners' FP32 distances are opposite
+ * to rounding (each side rounds its own shifted position), so the forces sum
+ * to zero to FP32 rounding; energy, virial and counts are taken on the task's
+ * i side only.
  */
 #include <hip/hip_runtime.h>
 
@@ -143,33 +142,6 @@ __device__ __forceinline__ float4 ld_f4(__amdgpu_buffer_rsrc_t r, int byte_off) 
     float4 out;
     __builtin_memcpy(&out, &v, sizeof(out));
     return out;
-}
-
-/* pot_eval32 with the coefficients behind a buffer resource. */
-__device__ __forceinline__ void pot_eval32r(const float4 hdr, __amdgpu_buffer_rsrc_t rc, float r2, float &e,
-                                            float &f) {
-    const float ir = __builtin_amdgcn_rsqf(r2);
-    const float r = r2 * ir;
-    const float fi = fmaxf(0.0f, hdr.x + r * (hdr.y + r * hdr.z));
-    const unsigned int w = __float_as_uint(hdr.w);
-    const int n = (int)(w & 511u);
-    int ind = (int)fi;
-    ind = ind > n ? n : ind;
-    const int off = 32 * ((int)(w >> 9) + ind);
-    const float4 a = ld_f4(rc, off), b = ld_f4(rc, off + 16);
-    const float x = (r - a.x) * a.y;
-    float ee = a.z * x + a.w;
-    float eff = a.z;
-    eff = eff * x + ee;
-    ee = ee * x + b.x;
-    eff = eff * x + ee;
-    ee = ee * x + b.y;
-    eff = eff * x + ee;
-    ee = ee * x + b.z;
-    eff = eff * x + ee;
-    ee = ee * x + b.w;
-    e = ee;
-    f = eff * a.y * ir;
 }
 
 /* pot_eval32r for two pairs at once, without branches: both coefficient
@@ -345,7 +317,8 @@ __global__ __launch_bounds__(256) void k_sort(struct nb_params P, const int *__r
                                               const int *__restrict__ offset,
                                               const unsigned int *__restrict__ sortflags,
                                               const double *__restrict__ x, unsigned int *__restrict__ sortlist,
-                                              unsigned short *__restrict__ keyof, int *__restrict__ flag) {
+                                              unsigned short *__restrict__ keyof,
+                                              unsigned short *__restrict__ kminmax, int *__restrict__ flag) {
     int t = blockIdx.x * blockDim.x + threadIdx.x;
     int cid = t / 13, sid = t - 13 * (t / 13);
     if (cid >= P.ncells) return;
@@ -361,6 +334,8 @@ __global__ __launch_bounds__(256) void k_sort(struct nb_params P, const int *__r
         keyof[(size_t)sid * P.nparts + off + i] = (unsigned short)key;
     }
     sort_desc(list, n, flag);
+    kminmax[26 * (size_t)cid + sid] = (unsigned short)(list[0] & 0xffffu);
+    kminmax[26 * (size_t)cid + 13 + sid] = (unsigned short)(list[n - 1] & 0xffffu);
 }
 
 /* The quicksort of sort_desc_t, run by a whole wave on one LDS list with the
@@ -753,7 +728,8 @@ __global__ __launch_bounds__(1024) void k_sort_rank(struct nb_params P, const in
                                                   const int *__restrict__ offset,
                                                   const unsigned int *__restrict__ sortflags,
                                                   const double *__restrict__ x, unsigned int *__restrict__ sortlist,
-                                                  unsigned short *__restrict__ keyof, int *__restrict__ flag,
+                                                  unsigned short *__restrict__ keyof,
+                                                  unsigned short *__restrict__ kminmax, int *__restrict__ flag,
                                                   int maxn) {
     extern __shared__ double sh_rank[];
     double *xs = sh_rank;
@@ -789,6 +765,9 @@ __global__ __launch_bounds__(1024) void k_sort_rank(struct nb_params P, const in
             gt += kj > key;
             eq += kj == key;
         }
+        /* largest and smallest key (particles that share one write the same) */
+        if (gt == 0) kminmax[26 * (size_t)c + sid] = (unsigned short)key;
+        if (gt + eq == n) kminmax[26 * (size_t)c + 13 + sid] = (unsigned short)key;
         if (eq == 1) {
             out[sid * n + gt] = w;
         } else {
@@ -840,10 +819,9 @@ struct nb_out {
     float4 *fhi, *flo;
     double *cell_acc;
     unsigned long long *cell_cnt;
-    /* half-shell mode: per visit (neighbour-list entry), the forces on the
-       visited cell's atoms, jcap slots per entry */
-    float4 *jpart;
-    int jcap;
+    /* half shell: forces on the visited atoms, jpart[slot][atom][3], slot 0 for
+       the self task and 1.. for the atom's cell's incoming tasks */
+    float *jpart;
     /* split owners (nsplit > 1): group g's forces on atom a at [g * nparts + a] */
     float4 *phi, *plo;
 };
@@ -925,15 +903,19 @@ __device__ __forceinline__ void mlp_dense_eval(const struct mlp_net &N, const fl
     }
 }
 
+#define MD_SPLIT_ITEMS_PER_CU 32 /* surrogate: work items per CU below which owners are split */
+#define MD_SPLIT_MAX 8           /* surrogate: at most this many neighbour groups per owner cell */
+#define MD_PAIR_ITEMS_PER_CU 12  /* k_pair: work items per CU that owners are split up to */
+#define MD_PAIR_SPLIT_MAX 32     /* k_pair: at most this many groups (of two entries at least) */
+#define MD_PAIR_R64_MEAN 32      /* atoms per cell above which k_pair takes 64 owner atoms at a time */
 #define MD_HCAP 32     /* table mode: hits buffered per lane before they are evaluated */
-#define MD_HCAP_WIDE 28 /* the same in the 5-wave builds: their LDS then allows 20 waves per CU */
-#define MD_SPLIT_ITEMS_PER_CU 32 /* pair-kernel work items per CU below which owners are split */
-#define MD_SPLIT_MAX 8           /* at most this many neighbour groups per owner cell */
+#define MD_HCAP_WIDE 28 /* the same in the 5-wave build: its LDS then allows 20 waves per CU */
 #define MD_HCAP_MLP 8  /* MLP mode: hits per lane per compaction round */
 #define MD_XCAP_MLP 8  /* MLP mode: excluded partners per lane per round */
 
-/* The pair kernel body, for both evaluation modes:
-   MLP = false  every hit is evaluated from the FP32 tables by its lane;
+/* The body of the kernels that walk the sorted windows, for two modes:
+   MLP = false  (half shell only) every hit is evaluated from the FP32 tables
+                by its lane;
    MLP = true   hits below the species pair's r_lo (or without a network)
                 are evaluated from the tables, the others are compacted
                 wave-wide into a dense LDS pair list and evaluated by the
@@ -941,7 +923,7 @@ __device__ __forceinline__ void mlp_dense_eval(const struct mlp_net &N, const fl
                 adds its own contiguous run of results in order, so the
                 result stays deterministic.  Excluded pairs take the same
                 route, so a pair and its exclusion cancel exactly. */
-template <bool MLP, bool HALF, bool PAIRED = false, bool REFCNT = true, int HC = MD_HCAP>
+template <bool MLP, bool HALF, int HC = MD_HCAP>
 __device__ __forceinline__ void nonbond_body(
     unsigned char *smem, struct nb_params P, const int2 *__restrict__ cnt_off, const int4 *__restrict__ nbr,
     const int *__restrict__ nbr_off, const float4 *__restrict__ nbs, const double *__restrict__ origin,
@@ -957,14 +939,14 @@ __device__ __forceinline__ void nonbond_body(
     int *kfl = (int *)(smem + P.lds_kfl);                                /* [26]        */
     float4 *stage = (float4 *)(smem + P.lds_stage);                      /* [maxn]      */
     unsigned short *hitl = (unsigned short *)(smem + P.lds_hit);         /* [HCAP*64]   */
-    /* MLP mode: dense pair list (r^2, species pair) and its results (f, e),
+    /* Dense pair list (r^2, species pair) and its results (f, e),
        and the excluded partners of each lane. */
     float *dn_r2 = (float *)(smem + P.lds_dense);                        /* [HCAP*64]   */
     int *dn_p = (int *)(smem + P.lds_dense + 4 * 64 * MD_HCAP_MLP);
     float *dn_f = (float *)(smem + P.lds_dense + 8 * 64 * MD_HCAP_MLP);
     float *dn_e = (float *)(smem + P.lds_dense + 12 * 64 * MD_HCAP_MLP);
     int *exb = (int *)(smem + P.lds_dense + 16 * 64 * MD_HCAP_MLP);      /* [XCAP*64]   */
-    /* MLP mode: layer 1's weights [64][2], copied once per wave */
+    /* layer 1's weights [64][2], copied once per wave */
     float *w1s = (float *)(smem + P.lds_dense + 16 * 64 * MD_HCAP_MLP + 4 * 64 * MD_XCAP_MLP);
     /* half-shell mode: forces on the visited cell's records, 3 per record */
     float *jf = (float *)(smem + P.lds_jf);                              /* [4][3*maxn] */
@@ -1049,77 +1031,39 @@ __device__ __forceinline__ void nonbond_body(
                     own_key[sid * 64 + lane] = keyof[(size_t)sid * P.nparts + offc + i0 + lane];
             wave_lds_sync();
 
-            /* Visits: one neighbour entry or, in the paired kernels, the two
-               entries of opposite offsets +d and -d, which share the sort
-               direction and so the owner's keys.  The first of the two is the
-               one whose pair task has the owner as its i cell (bit 6 marks
-               it, bit 7 its partner).  The owner atoms' windows into the two
-               cells are long and short in turn, so that each lane's walk
-               through both is about as long as any other's.  Segment A of
-               the staged records is the first entry's cell, segment B the
-               second's. */
-            int kbeg = 0;
-            if constexpr (PAIRED)
-                if (nn > 0 && (nbr[k0].y & 128)) kbeg = 1; /* opened by its partner in the previous group */
-
-            /* Prefetch a visit's first 64 staged positions: lane t < nA holds
-               atom t of A (unsorted position) and A's window word t, lane
-               nA + u the same for atom u of B. */
+            /* Prefetch a visit's first 64 staged positions: lane t holds atom t
+               of the neighbour cell (unsorted position) and its window word t. */
             float4 pfx = make_float4(0.f, 0.f, 0.f, 0.f);
             unsigned int pfw = 0;
             auto prefetch = [&](int kv) {
-                const int4 ea = nbr[k0 + kv];
-                const int2 ca = cnt_off[ea.x];
-                bool sB = false;
-                int2 cs = ca;
-                int4 es = ea;
-                if constexpr (PAIRED) {
-                    if (ea.y & 64) {
-                        const int4 eb = nbr[k0 + kv + 1];
-                        const int2 cb = cnt_off[eb.x];
-                        sB = lane >= ca.x;
-                        cs = sB ? cb : ca;
-                        es = sB ? eb : ea;
-                    }
-                }
-                const int u = sB ? lane - ca.x : lane;
-                if (u < cs.x) {
-                    pfx = xf[cs.y + u];
-                    if (!(es.y & 32)) {
-                        const int sid = es.y & 15, orient = (es.y >> 4) & 1;
-                        pfw = sortlist[13 * (size_t)cs.y + (size_t)sid * cs.x + (orient ? u : cs.x - 1 - u)];
+                const int4 en = nbr[k0 + kv];
+                const int2 cs = cnt_off[en.x];
+                if (lane < cs.x) {
+                    pfx = xf[cs.y + lane];
+                    if (!(en.y & 32)) {
+                        const int sid = en.y & 15, orient = (en.y >> 4) & 1;
+                        pfw = sortlist[13 * (size_t)cs.y + (size_t)sid * cs.x + (orient ? lane : cs.x - 1 - lane)];
                     }
                 }
             };
-            if (kbeg < nn) prefetch(kbeg);
+            if (nn > 0) prefetch(0);
 
             float hx = 0.f, hy = 0.f, hz = 0.f, lx = 0.f, ly = 0.f, lz = 0.f;
             double epot = 0.0, vir = 0.0, eexcl = 0.0;
             unsigned int np = 0, nref = 0, nexcl = 0;
 
-            for (int k = kbeg, step = 1; k < nn; k += step) {
+            for (int k = 0; k < nn; k++) {
                 const int4 en = nbr[k0 + k];
-                const bool paired = PAIRED && (en.y & 64);
-                step = paired ? 2 : 1;
-                const int4 enb = paired ? nbr[k0 + k + 1] : en;
                 const int2 cjc = cnt_off[en.x];
-                const int cj = en.x, nA = cjc.x, offj = cjc.y;
-                int nB = 0, offB = 0;
-                if (paired) {
-                    const int2 cb = cnt_off[enb.x];
-                    nB = cb.x;
-                    offB = cb.y;
-                }
-                const int nj = nA + nB;
+                const int cj = en.x, nj = cjc.x, offj = cjc.y;
                 const int sid = en.y & 15, orient = (en.y >> 4) & 1, self = (en.y >> 5) & 1;
 
-                /* Shifts from the owner cell to the neighbours (minimum image),
+                /* Shift from the owner cell to the neighbour (minimum image),
                    rounded to FP32 on the host; the FP64 value is recomputed
                    where needed. */
                 const float4 sfv = nbs[k0 + k];
-                const float4 sgv = paired ? nbs[k0 + k + 1] : sfv;
 
-                /* Stage the neighbours, each in the order its window is
+                /* Stage the neighbour in the order its window is
                    walked: ascending keys when the owner is the task's i cell,
                    descending otherwise, storage order for the self task.
                    Record = (x + s, y + s, z + s, key' | index << 16 | type << tshift):
@@ -1131,22 +1075,18 @@ __device__ __forceinline__ void nonbond_body(
                 if (lane < nj) raw[lane] = pfx;
                 wave_lds_sync();
                 for (int t = lane; t < nj; t += 64) {
-                    const bool sB = t >= nA;
-                    const int u = sB ? t - nA : t, ns = sB ? nB : nA, os = sB ? offB : offj, rb = sB ? nA : 0;
-                    const int ori = sB ? 1 : orient;
-                    const float4 sh = sB ? sgv : sfv;
                     if (self) {
                         const float4 p = t < 64 ? pfx : xf[offj + t];
-                        stage[t] = make_float4(p.x + sh.x, p.y + sh.y, p.z + sh.z,
+                        stage[t] = make_float4(p.x + sfv.x, p.y + sfv.y, p.z + sfv.z,
                                                __uint_as_float(((unsigned int)t << 16) |
                                                                ((unsigned int)__float_as_int(p.w) << P.tshift)));
                     } else {
                         const unsigned int w =
-                            t < 64 ? pfw : sortlist[13 * (size_t)os + (size_t)sid * ns + (ori ? u : ns - 1 - u)];
-                        const int idx = (int)(w >> 16) < ns ? (int)(w >> 16) : ns - 1;
-                        const float4 p = rb + idx < 64 ? raw[rb + idx] : xf[os + idx];
-                        const unsigned int kk = ori ? 0xffffu - (w & 0xffffu) : (w & 0xffffu);
-                        stage[t] = make_float4(p.x + sh.x, p.y + sh.y, p.z + sh.z,
+                            t < 64 ? pfw : sortlist[13 * (size_t)offj + (size_t)sid * nj + (orient ? t : nj - 1 - t)];
+                        const int idx = (int)(w >> 16) < nj ? (int)(w >> 16) : nj - 1;
+                        const float4 p = idx < 64 ? raw[idx] : xf[offj + idx];
+                        const unsigned int kk = orient ? 0xffffu - (w & 0xffffu) : (w & 0xffffu);
+                        stage[t] = make_float4(p.x + sfv.x, p.y + sfv.y, p.z + sfv.z,
                                                __uint_as_float(kk | ((unsigned int)idx << 16) |
                                                                ((unsigned int)__float_as_int(p.w) << P.tshift)));
                     }
@@ -1154,34 +1094,22 @@ __device__ __forceinline__ void nonbond_body(
                 wave_lds_sync();
 
                 /* Prefetch the next visit while this one is processed. */
-                if (k + step < nn) prefetch(k + step);
+                if (k + 1 < nn) prefetch(k + 1);
                 if (nj == 0) continue;
 
                 int myk = 0, dns = 0;
                 bool live_ref = true, run = true;
                 if (!self) {
                     dns = P.proj ? en.w : en.z;
-                    if (nA > 0) {
+                    {
                         const int kr = (int)(__float_as_uint(stage[0].w) & 0xffffu);
                         const int kstage0 = orient ? 0xffff - kr : kr; /* staged keys are complemented when orient */
                         const int s_imax = orient ? kstage0 : kfl[sid];
                         const int s_jmin = orient ? kfl[13 + sid] : kstage0;
                         live_ref = (s_jmin + en.z - s_imax) >= 0;
                         run = P.proj || live_ref;
-                    } else {
-                        live_ref = run = false;
                     }
                     myk = own_key[sid * 64 + il];
-                }
-                /* Segment B: the owner is the j cell of its task. */
-                int kmaxB = 0;
-                bool runB = false;
-                if (paired && nB > 0) {
-                    const int kr = (int)(__float_as_uint(stage[nA].w) & 0xffffu);
-                    runB = P.proj || (kfl[13 + sid] + enb.z - (0xffff - kr)) >= 0;
-                    const int dmdB = P.maxdx != nullptr ? pair_dmaxdist(P.dscale, P.cutoff, P.maxdx[enb.x], P.maxdx[c])
-                                                        : P.dmaxdist;
-                    kmaxB = dmdB - (myk + (P.proj ? enb.w : enb.z) - 0xffff);
                 }
                 /* Window (runner_dopair.c:455-478): record t is admitted while
                    key_j + dnshift - key_i < dmaxdist (owner is i) or
@@ -1313,14 +1241,14 @@ __device__ __forceinline__ void nonbond_body(
                                         le += ea;
                                         lv -= fa * r2a;
                                         lnp++;
-                                        if (REFCNT && P.proj) lnref += (VK == 0 ||
+                                        if (P.proj) lnref += (VK == 0 ||
                                                   (live_ref && ((int)rec_key(wa) + en.z - myk) < dmd)) ? 1u : 0u;
                                     }
                                     if (cb) {
                                         le += eb;
                                         lv -= fb * r2b;
                                         lnp++;
-                                        if (REFCNT && P.proj) lnref += (VK == 0 ||
+                                        if (P.proj) lnref += (VK == 0 ||
                                                   (live_ref && ((int)rec_key(wb) + en.z - myk) < dmd)) ? 1u : 0u;
                                     }
                                 }
@@ -1359,7 +1287,7 @@ __device__ __forceinline__ void nonbond_body(
                                     le += ea;
                                     lv -= fa * r2a;
                                     lnp++;
-                                    if (REFCNT && P.proj) lnref += (VK == 0 ||
+                                    if (P.proj) lnref += (VK == 0 ||
                                               (live_ref && ((int)rec_key(wa) + en.z - myk) < dmd)) ? 1u : 0u;
                                 }
                             }
@@ -1395,7 +1323,7 @@ __device__ __forceinline__ void nonbond_body(
                                     le += ea;
                                     lv -= fa * r2a;
                                     lnp++;
-                                    if (REFCNT && P.proj) lnref += (VK == 0 ||
+                                    if (P.proj) lnref += (VK == 0 ||
                                               (live_ref && ((int)rec_key(wa) + en.z - myk) < dmd)) ? 1u : 0u;
                                 }
                             }
@@ -1403,94 +1331,12 @@ __device__ __forceinline__ void nonbond_body(
                         }
                     }
                 };
-                /* A paired visit: each lane walks its share of its atom's window
-                   in A (the owner is the i cell: energies, virial and counts
-                   are taken there), then, from its first record past that
-                   window, its share of the window in B (forces only). */
-                auto visit_pair = [&]() {
-                    int t = part, seg = run ? 0 : 1;
-                    bool alive = active && (run || runB);
-                    while (wave_any(alive)) {
-                        int h = 0;
-                        for (int it = 0; it < HCAP; it++) {
-                            const int base = seg ? nA : 0, ns = seg ? nB : nA, km = seg ? kmaxB : kmax;
-                            const int tt = base + (t < ns ? t : (ns > 0 ? ns - 1 : 0));
-                            const float4 pj = stage[tt];
-                            const unsigned int wj = __float_as_uint(pj.w);
-                            const bool inwin = alive && t < ns && (int)rec_key(wj) < km;
-                            const bool sw = alive && !inwin && seg == 0;
-                            alive = inwin || (sw && runB);
-                            const float dx = xi.x - pj.x, dy = xi.y - pj.y, dz = xi.z - pj.z;
-                            const float r2 = dx * dx + dy * dy + dz * dz;
-                            const bool hit = inwin && r2 <= rc2hi;
-                            hitl[h * 64 + lane] = (unsigned short)tt;
-                            h += hit ? 1 : 0;
-                            if (sw) {
-                                t = part;
-                                seg = 1;
-                            } else if (inwin)
-                                t += NPi;
-                            if (!wave_any(alive)) break;
-                        }
-                        /* Evaluate the kept hits, two per lane per round. */
-                        for (int s = 0; wave_any(s < h); s += 2) {
-                            const bool va = s < h, vb = s + 1 < h;
-                            const int ta = va ? hitl[s * 64 + lane] : 0;
-                            const int tb = vb ? hitl[(s + 1) * 64 + lane] : ta;
-                            const float4 pa = stage[ta], pb = stage[tb];
-                            const unsigned int wa = __float_as_uint(pa.w), wb = __float_as_uint(pb.w);
-                            const float4 ha = ld_f4(rs_ptab, 16 * (ti * mt + rec_type(wa, P.tshift)));
-                            const float4 hb = ld_f4(rs_ptab, 16 * (ti * mt + rec_type(wb, P.tshift)));
-                            const bool ia = ta < nA, ib = tb < nA;
-                            const float dxa = xi.x - pa.x, dya = xi.y - pa.y, dza = xi.z - pa.z;
-                            const float dxb = xi.x - pb.x, dyb = xi.y - pb.y, dzb = xi.z - pb.z;
-                            const float r2a = dxa * dxa + dya * dya + dza * dza;
-                            const float r2b = dxb * dxb + dyb * dyb + dzb * dzb;
-                            bool ua = va && __float_as_int(ha.w) != -1;
-                            bool ub = vb && __float_as_int(hb.w) != -1;
-                            const bool na = ua && fabsf(r2a - P.rc2f) <= P.band;
-                            const bool nb = ub && fabsf(r2b - P.rc2f) <= P.band;
-                            if (wave_any(na || nb)) {
-                                if (na) ua = ia ? in_cut64(cj, offj, wa, true) : in_cut64(enb.x, offB, wa, false);
-                                if (nb) ub = ib ? in_cut64(cj, offj, wb, true) : in_cut64(enb.x, offB, wb, false);
-                            }
-                            float ea, fa, eb, fb;
-                            pot_eval32r2(ha, hb, ua, ub, rs_coef, r2a, r2b, ea, fa, eb, fb);
-                            lfx = fmaf(-fb, dxb, fmaf(-fa, dxa, lfx));
-                            lfy = fmaf(-fb, dyb, fmaf(-fa, dya, lfy));
-                            lfz = fmaf(-fb, dzb, fmaf(-fa, dza, lfz));
-                            if (ua && ia) {
-                                le += ea;
-                                lv -= fa * r2a;
-                                lnp++;
-                                if (REFCNT && P.proj) lnref += (live_ref && ((int)rec_key(wa) + en.z - myk) < dmd) ? 1u : 0u;
-                            }
-                            if (ub && ib) {
-                                le += eb;
-                                lv -= fb * r2b;
-                                lnp++;
-                                if (REFCNT && P.proj) lnref += (live_ref && ((int)rec_key(wb) + en.z - myk) < dmd) ? 1u : 0u;
-                            }
-                        }
-                    }
-                };
-                if constexpr (PAIRED) {
-                    if (paired)
-                        visit_pair();
-                    else if (self)
-                        visit(visit_kind<0>{});
-                    else if (orient == 0)
-                        visit(visit_kind<1>{});
-                    else
-                        visit(visit_kind<2>{});
-                } else {
-                    if (self)
-                        visit(visit_kind<0>{});
-                    else if (orient == 0)
-                        visit(visit_kind<1>{});
-                    else
-                        visit(visit_kind<2>{});
-                }
+                if (self)
+                    visit(visit_kind<0>{});
+                else if (orient == 0)
+                    visit(visit_kind<1>{});
+                else
+                    visit(visit_kind<2>{});
                 if constexpr (HALF) {
                     /* this visit's forces on the visited atoms, by slot; later
                        chunks of the owner add to the first one's */
@@ -1505,13 +1351,8 @@ __device__ __forceinline__ void nonbond_body(
                             vv[m] = (j0[0] + j0[s]) + (j0[2 * s] + j0[3 * s]);
                             j0[0] = j0[s] = j0[2 * s] = j0[3 * s] = 0.f;
                         }
-                        float4 v = make_float4(vv[0], vv[1], vv[2], 0.f);
-                        float4 *dst = &O.jpart[(size_t)(k0 + k) * O.jcap + idx];
-                        if (ch > 0) {
-                            const float4 o = *dst;
-                            v = make_float4(o.x + v.x, o.y + v.y, o.z + v.z, 0.f);
-                        }
-                        *dst = v;
+                        float *dst = O.jpart + 3 * ((size_t)((unsigned int)en.y >> 9) * P.nparts + offj + idx);
+                        for (int m = 0; m < 3; m++) dst[m] = ch > 0 ? dst[m] + vv[m] : vv[m];
                     }
                 }
                 acc2(hx, lx, lfx);
@@ -1520,7 +1361,7 @@ __device__ __forceinline__ void nonbond_body(
                 epot += (double)le;
                 vir += (double)lv;
                 np += lnp;
-                nref += (REFCNT && P.proj) ? lnref : lnp;
+                nref += P.proj ? lnref : lnp;
             }
 
             /* Excluded pairs: subtract what the pair pass added
@@ -1697,6 +1538,8 @@ __device__ __forceinline__ void nonbond_body(
     }
 }
 
+#include "pair_tile.h"
+
 #define NB_PARAMS                                                                                             \
     struct nb_params P, const int2 *__restrict__ cnt_off, const int4 *__restrict__ nbr,                       \
         const int *__restrict__ nbr_off, const float4 *__restrict__ nbs, const double *__restrict__ origin,   \
@@ -1710,39 +1553,25 @@ __device__ __forceinline__ void nonbond_body(
     P, cnt_off, nbr, nbr_off, nbs, origin, loc, xf, x64, pid, sortlist, keyof, ptab, coeffs4, excl_off, excl_list, \
         index_of_id, cell_of, O, queue
 
-/* Table mode.  The occupancy hint keeps it at 4 waves per SIMD (128
-   VGPRs); the kernel is bound by instruction issue and latency, and 4 waves
-   measured faster than 3 without the hint. */
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_nonbond(NB_PARAMS) {
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    const struct mlp_net N = {};
-    nonbond_body<false, false>(smem, NB_ARGS, N, nullptr);
-}
+/* Table mode, full shell (pair_tile.h): at most 32 or 64 owner atoms at a
+   time, the reference's or the projected window. */
+#define PAIR_PARAMS                                                                                           \
+    struct nb_params P, const int2 *__restrict__ cnt_off, const int4 *__restrict__ nbr,                       \
+        const int *__restrict__ nbr_off, const int *__restrict__ nbr_mid, const float4 *__restrict__ nbs,     \
+        const double *__restrict__ origin, const int *__restrict__ loc,                                      \
+        const float4 *__restrict__ xf, const double *__restrict__ x64, const int *__restrict__ pid,          \
+        const unsigned short *__restrict__ kminmax, const unsigned int *__restrict__ sortlist,                \
+        const unsigned short *__restrict__ keyof, const float4 *__restrict__ ptab,                           \
+        const float4 *__restrict__ coeffs4, const int *__restrict__ excl_off, const int *__restrict__ excl_list, \
+        const int *__restrict__ index_of_id, const int *__restrict__ cell_of, struct nb_out O
+#define PAIR_ARGS                                                                                             \
+    P, cnt_off, nbr, nbr_off, nbr_mid, nbs, origin, loc, xf, x64, pid, kminmax, sortlist, keyof, ptab, \
+        coeffs4, excl_off, excl_list, index_of_id, cell_of, O
 
-/* Table mode with paired visits (neighbour cells at opposite offsets
-   together), under the 4- and the 5-wave register budgets.  Reference
-   window only: they do not count the pairs the reference window would
-   admit (with the reference window that count is the pair count). */
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_nonbond_paired(NB_PARAMS) {
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    const struct mlp_net N = {};
-    nonbond_body<false, false, true, false>(smem, NB_ARGS, N, nullptr);
-}
-
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_nonbond_paired_wide(NB_PARAMS) {
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    const struct mlp_net N = {};
-    nonbond_body<false, false, true, false, MD_HCAP_WIDE>(smem, NB_ARGS, N, nullptr);
-}
-
-/* Table mode for systems with many more cells than resident waves: the same
-   body under a 96-register budget (5 waves per SIMD), which pays off when
-   every wave has cells to take; with few cells per wave the 4-wave build's
-   lower latency per cell wins. */
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_nonbond_wide(NB_PARAMS) {
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    const struct mlp_net N = {};
-    nonbond_body<false, false, false, true, MD_HCAP_WIDE>(smem, NB_ARGS, N, nullptr);
+template <int R, bool PROJ>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(R == 32 ? 4 : 3, 8))) void k_pair(PAIR_PARAMS) {
+    __shared__ __attribute__((aligned(16))) pair_lds<R> L;
+    pair_body<R, PROJ>(L, PAIR_ARGS);
 }
 
 /* Surrogate mode (engine_flag_mlp). */
@@ -1757,8 +1586,8 @@ __global__ __launch_bounds__(64) void k_nonbond_mlp_half(NB_PARAMS, struct mlp_n
     nonbond_body<true, true>(smem, NB_ARGS, N, ptype);
 }
 
-/* Half shell: each pair task once, from its i cell, with the opposite
-   forces on the j cell's atoms left per visit for k_fold. */
+/* Table mode on the half shell: each pair once, at the i cell of its task.
+   The 5-wave build is for many cells. */
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_nonbond_half(NB_PARAMS) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const struct mlp_net N = {};
@@ -1767,23 +1596,24 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_nonbond_half_wide(NB_PARAMS) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const struct mlp_net N = {};
-    nonbond_body<false, true>(smem, NB_ARGS, N, nullptr);
+    nonbond_body<false, true, MD_HCAP_WIDE>(smem, NB_ARGS, N, nullptr);
 }
 
 /* Second step of a split and/or half-shell pass, one wave per cell: each
    atom's force = its owner's (hi, lo), or with nsplit > 1 the groups'
-   (hi, lo) in group order, plus (half shell) the forces its cell received as
-   the j cell of other cells' tasks and in its own self task, in a fixed
-   order (the self entry, then the incoming entries in ascending order),
-   all added with two-sum. */
+   (hi, lo) in group order, plus (half shell) the forces its cell received in
+   its own self task (slot 0) and as the j cell of other cells' tasks (slots
+   1.. in task order, those of empty i cells left out: nothing writes them),
+   all added with two-sum in that order.  Reads as a stream: the slots of
+   consecutive atoms are consecutive, and 8 are in flight per lane. */
 __global__ __launch_bounds__(64) void k_fold(int ncells, const int2 *__restrict__ cnt_off, int nsplit, int nparts,
                                              const float4 *__restrict__ phi, const float4 *__restrict__ plo, int half,
-                                             const int *__restrict__ self_entry, const int *__restrict__ inv_off,
-                                             const int *__restrict__ inv_list, const float4 *__restrict__ jpart,
-                                             int jcap, float4 *__restrict__ fhi, float4 *__restrict__ flo) {
+                                             const int *__restrict__ inv_off, const int *__restrict__ inv_cell,
+                                             const float *__restrict__ jpart, float4 *__restrict__ fhi,
+                                             float4 *__restrict__ flo) {
     const int c = blockIdx.x, lane = threadIdx.x;
     const int2 co = cnt_off[c];
-    const int q0 = half ? inv_off[c] : 0, q1 = half ? inv_off[c + 1] : 0, es = half ? self_entry[c] : -1;
+    const int q0 = half ? inv_off[c] : 0, nq = half ? inv_off[c + 1] - q0 + 1 : 0;
     for (int s = lane; s < co.x; s += 64) {
         const int a = co.y + s;
         const float4 h = nsplit > 1 ? phi[a] : fhi[a], l = nsplit > 1 ? plo[a] : flo[a];
@@ -1797,17 +1627,22 @@ __global__ __launch_bounds__(64) void k_fold(int ncells, const int2 *__restrict_
             ly += ol.y;
             lz += ol.z;
         }
-        if (es >= 0) {
-            const float4 v = jpart[(size_t)es * jcap + s];
-            acc2(hx, lx, v.x);
-            acc2(hy, ly, v.y);
-            acc2(hz, lz, v.z);
-        }
-        for (int q = q0; q < q1; q++) {
-            const float4 v = jpart[(size_t)inv_list[q] * jcap + s];
-            acc2(hx, lx, v.x);
-            acc2(hy, ly, v.y);
-            acc2(hz, lz, v.z);
+        for (int q = 0; q < nq; q += 8) {
+            float v[8][3];
+#pragma unroll
+            for (int m = 0; m < 8; m++) {
+                const bool in = q + m < nq && (q + m == 0 || cnt_off[inv_cell[q0 + q + m - 1]].x > 0);
+                const float *src = jpart + 3 * ((size_t)(q + m) * nparts + a);
+                v[m][0] = in ? src[0] : 0.f;
+                v[m][1] = in ? src[1] : 0.f;
+                v[m][2] = in ? src[2] : 0.f;
+            }
+#pragma unroll
+            for (int m = 0; m < 8; m++) {
+                acc2(hx, lx, v[m][0]);
+                acc2(hy, ly, v[m][1]);
+                acc2(hz, lz, v[m][2]);
+            }
         }
         fhi[a] = make_float4(hx, hy, hz, 0.0f);
         flo[a] = make_float4(lx, ly, lz, 0.0f);
@@ -1986,14 +1821,13 @@ extern "C" int engine_gpu_finalize(struct engine *e) {
     (void)hipFree(g->d_nbr);
     (void)hipFree(g->d_nbs);
     (void)hipFree(g->d_nbr_off);
-    (void)hipFree(g->d_nbr_p);
-    (void)hipFree(g->d_nbs_p);
+    (void)hipFree(g->d_nbr_mid);
+    (void)hipFree(g->d_kminmax);
     (void)hipFree(g->d_nbr_h);
     (void)hipFree(g->d_nbs_h);
     (void)hipFree(g->d_nbr_off_h);
-    (void)hipFree(g->d_self_entry);
     (void)hipFree(g->d_inv_off);
-    (void)hipFree(g->d_inv_list);
+    (void)hipFree(g->d_inv_cell);
     (void)hipFree(g->d_jpart);
     (void)hipFree(g->d_phi);
     (void)hipFree(g->d_plo);
@@ -2028,19 +1862,19 @@ extern "C" int engine_gpu_finalize(struct engine *e) {
     return engine_err_ok;
 }
 
-/* FP32 minimum-image shift from cell a's origin to cell b's: the same FP64
-   arithmetic as min_image() on the device, rounded once. */
+/* Minimum-image shift from cell a's origin to cell b's: the same FP64
+   arithmetic as min_image() on the device, rounded once to FP32. */
 static float4 cell_shift32(const struct space *s, int a, int b) {
-    float v[3];
+    double v[3];
     for (int k = 0; k < 3; k++) {
         double d = s->cells[b].origin[k] - s->cells[a].origin[k];
         if (d * 2 > s->dim[k])
             d -= s->dim[k];
         else if (d * 2 < -s->dim[k])
             d += s->dim[k];
-        v[k] = (float)d;
+        v[k] = d;
     }
-    return make_float4(v[0], v[1], v[2], 0.f);
+    return make_float4((float)v[0], (float)v[1], (float)v[2], 0.f);
 }
 
 /* dnshift of a pair task (runner_dopair.c:426-452): with the reference's
@@ -2060,6 +1894,15 @@ static void task_dnshift(const struct space *s, int ti, int tj, int sid, double 
     *dns_ref = (int)(dscale * nshift);
     dot = sh[0] * cell_shift[3 * sid] + sh[1] * cell_shift[3 * sid + 1] + sh[2] * cell_shift[3 * sid + 2];
     *dns_proj = (int)(dscale * dot);
+}
+
+/* Whether a task needs the window test: the reference window may cut pairs
+   within the cutoff.  Not so when the offset lies along the sort axis
+   (pair_tile.h), unless dscale rc is so close below an integer that the
+   rounding of the keys' FP64 arithmetic (~1e-11) could matter. */
+static int task_window(const struct gpu_state *g, const struct space *s, int dns_ref, int dns_proj) {
+    const double rcd = g->P.dscale * s->cutoff;
+    return dns_ref > dns_proj || rcd - floor(rcd) > 1.0 - 1e-9;
 }
 
 extern "C" int engine_gpu_load(struct engine *e) {
@@ -2186,6 +2029,15 @@ extern "C" int engine_gpu_load(struct engine *e) {
             g->maxcell = 1 << (16 - tbits);
         }
         P->maxdx = NULL;
+        P->window = 0;
+        /* k_pair's filter threshold: above the cutoff band by 16 roundings
+           of the largest squared coordinate in an owner's frame (the four
+           products, their sum and |x|^2 stay below 8 of them) */
+        {
+            double r2 = 0.0;
+            for (k = 0; k < 3; k++) r2 += (s->span[k] + 2) * s->h[k] * (s->span[k] + 2) * s->h[k];
+            P->filt = (float)(s->cutoff * s->cutoff * (1.0 + 2.1e-5) + r2 * 16.0 / 16777216.0);
+        }
         P->cutoff2 = s->cutoff * s->cutoff;
         for (k = 0; k < 3; k++) {
             P->dim[k] = s->dim[k];
@@ -2225,6 +2077,11 @@ extern "C" int engine_gpu_load(struct engine *e) {
         for (cid = 0; cid < s->nr_cells; cid++) fill[cid + 1] = fill[cid] + cnt[cid];
         memcpy(off, fill, sizeof(int) * (s->nr_cells + 1));
         nbs = (float4 *)malloc(sizeof(float4) * (total > 0 ? total : 1));
+        /* the cells' distance class of an entry, its square in cells, goes
+           along in bits 16 and up */
+        const float ih[3] = {(float)(1.0 / s->h[0]), (float)(1.0 / s->h[1]), (float)(1.0 / s->h[2])};
+        const int ND = 256;
+        int nd = 1; /* distance classes in use */
         for (k = 0; k < s->nr_tasks; k++) {
             struct task *t = &s->tasks[k];
             if (t->type == task_type_self) {
@@ -2233,11 +2090,64 @@ extern "C" int engine_gpu_load(struct engine *e) {
             } else if (t->type == task_type_pair) {
                 int dr, dp;
                 task_dnshift(s, t->i, t->j, t->flags, g->P.dscale, &dr, &dp);
-                nbs[fill[t->i]] = cell_shift32(s, t->i, t->j);
-                nbr[fill[t->i]++] = make_int4(t->j, t->flags, dr, dp);
-                nbs[fill[t->j]] = cell_shift32(s, t->j, t->i);
-                nbr[fill[t->j]++] = make_int4(t->i, t->flags | (1 << 4), dr, dp);
+                const int win = task_window(g, s, dr, dp) << 8;
+                if (win) g->P.window = 1;
+                const float4 sh = cell_shift32(s, t->i, t->j);
+                const float d[3] = {sh.x * ih[0], sh.y * ih[1], sh.z * ih[2]};
+                const int d2 = (int)(d[0] * d[0] + d[1] * d[1] + d[2] * d[2] + 0.5f);
+                const int dc = d2 < ND ? d2 : ND - 1;
+                const int y = t->flags | win | (dc << 16);
+                if (dc >= nd) nd = dc + 1;
+                nbs[fill[t->i]] = sh;
+                nbr[fill[t->i]++] = make_int4(t->j, y, dr, dp);
+                nbs[fill[t->j]] = make_float4(-sh.x, -sh.y, -sh.z, 0.f);
+                nbr[fill[t->j]++] = make_int4(t->i, y | (1 << 4), dr, dp);
             }
+        }
+        /* Per owner, the entries whose task has it as the i cell (the self
+           task the very first), then the others; of both those without a
+           window test first (k_pair's chunks then mostly need the test or do
+           not), and nearer cells first: a chunk's cells then hold about as
+           many hits for every owner atom. */
+        {
+            int4 *tn = (int4 *)malloc(sizeof(int4) * maxnbr);
+            float4 *ts = (float4 *)malloc(sizeof(float4) * maxnbr);
+            int *mid = (int *)malloc(sizeof(int) * s->nr_cells);
+            int bin[4 * ND];
+            if (tn == NULL || ts == NULL || mid == NULL) {
+                free(tn);
+                free(ts);
+                free(mid);
+                return gerror_(engine_err_malloc, "malloc failed");
+            }
+            auto cls = [nd, ND](const int4 &en) {
+                return (((en.y >> 4) & 1) * 2 + ((en.y >> 8) & 1)) * nd + ((en.y >> 16) & (ND - 1));
+            };
+            for (cid = 0; cid < s->nr_cells; cid++) {
+                const int b0 = off[cid], n = off[cid + 1] - off[cid];
+                memcpy(tn, &nbr[b0], sizeof(int4) * n);
+                memcpy(ts, &nbs[b0], sizeof(float4) * n);
+                memset(bin, 0, sizeof(int) * 4 * nd);
+                for (k = 0; k < n; k++) bin[cls(tn[k])]++;
+                for (int b = 0, m = b0; b < 4 * nd; b++) {
+                    if (b == 2 * nd) mid[cid] = m;
+                    const int c = bin[b];
+                    bin[b] = m;
+                    m += c;
+                }
+                for (k = 0; k < n; k++) {
+                    const int m = bin[cls(tn[k])]++;
+                    nbr[m] = tn[k];
+                    nbs[m] = ts[k];
+                }
+            }
+            free(tn);
+            free(ts);
+            const bool badm =
+                hipMalloc(&g->d_nbr_mid, sizeof(int) * s->nr_cells) != hipSuccess ||
+                hipMemcpy(g->d_nbr_mid, mid, sizeof(int) * s->nr_cells, hipMemcpyHostToDevice) != hipSuccess;
+            free(mid);
+            if (badm) return gerror_(engine_err_gpu, "neighbour lists");
         }
         g->maxnbr = maxnbr;
         g->P.maxnbr = maxnbr;
@@ -2247,88 +2157,6 @@ extern "C" int engine_gpu_load(struct engine *e) {
         HIPCHECK(hipMalloc(&g->d_nbs, sizeof(float4) * (total > 0 ? total : 1)));
         HIPCHECK(hipMemcpy(g->d_nbs, nbs, sizeof(float4) * (total > 0 ? total : 1), hipMemcpyHostToDevice));
         HIPCHECK(hipMemcpy(g->d_nbr_off, off, sizeof(int) * (s->nr_cells + 1), hipMemcpyHostToDevice));
-        /* Paired order: per owner the self entry, then each entry whose task
-           has the owner as its i cell followed by the entry at the opposite
-           cell offset with the same sort direction (the owner is its task's
-           j cell), then the entries left over, each list in task order. */
-        {
-            int4 *pn = (int4 *)malloc(sizeof(int4) * (total > 0 ? total : 1));
-            float4 *ps = (float4 *)malloc(sizeof(float4) * (total > 0 ? total : 1));
-            int *used = (int *)calloc(maxnbr + 1, sizeof(int));
-            int *slot = (int *)malloc(sizeof(int) * 17 * 17 * 17);
-            if (pn == NULL || ps == NULL || used == NULL || slot == NULL) {
-                free(pn);
-                free(ps);
-                free(used);
-                free(slot);
-                return gerror_(engine_err_malloc, "malloc failed");
-            }
-            for (k = 0; k < 17 * 17 * 17; k++) slot[k] = -1;
-            auto ofs_key = [&](const float4 v) {
-                int d[3];
-                const float sh[3] = {v.x, v.y, v.z};
-                for (int m = 0; m < 3; m++) {
-                    d[m] = (int)lrint(sh[m] / s->h[m]);
-                    d[m] = d[m] < -8 ? -8 : (d[m] > 8 ? 8 : d[m]);
-                }
-                return ((d[0] + 8) * 17 + (d[1] + 8)) * 17 + (d[2] + 8);
-            };
-            for (cid = 0; cid < s->nr_cells; cid++) {
-                const int b0 = off[cid], n = off[cid + 1] - off[cid];
-                int q = b0;
-                for (k = 0; k < n; k++) used[k] = 0;
-                /* the entries the owner is the j cell of, by cell offset */
-                for (k = 0; k < n; k++)
-                    if (!(nbr[b0 + k].y & 32) && (nbr[b0 + k].y & 16)) {
-                        const int key = ofs_key(nbs[b0 + k]);
-                        if (slot[key] < 0) slot[key] = k;
-                    }
-                for (k = 0; k < n; k++)
-                    if (nbr[b0 + k].y & 32) {
-                        pn[q] = nbr[b0 + k];
-                        ps[q++] = nbs[b0 + k];
-                        used[k] = 1;
-                    }
-                for (k = 0; k < n; k++) {
-                    const int4 ea = nbr[b0 + k];
-                    if (used[k] || (ea.y & 48)) continue;
-                    const float4 sa = nbs[b0 + k];
-                    const int key = ofs_key(make_float4(-sa.x, -sa.y, -sa.z, 0.f));
-                    const int m = slot[key];
-                    used[k] = 1;
-                    pn[q] = ea;
-                    ps[q++] = sa;
-                    if (m >= 0 && !used[m] && (nbr[b0 + m].y & 15) == (ea.y & 15)) {
-                        used[m] = 1;
-                        pn[q - 1].y |= 64;
-                        pn[q] = nbr[b0 + m];
-                        pn[q].y |= 128;
-                        ps[q++] = nbs[b0 + m];
-                    }
-                }
-                for (k = 0; k < n; k++)
-                    if (!used[k]) {
-                        pn[q] = nbr[b0 + k];
-                        ps[q++] = nbs[b0 + k];
-                    }
-                for (k = 0; k < n; k++)
-                    if (!(nbr[b0 + k].y & 32) && (nbr[b0 + k].y & 16)) slot[ofs_key(nbs[b0 + k])] = -1;
-            }
-            free(used);
-            free(slot);
-            if (hipMalloc(&g->d_nbr_p, sizeof(int4) * (total > 0 ? total : 1)) != hipSuccess ||
-                hipMalloc(&g->d_nbs_p, sizeof(float4) * (total > 0 ? total : 1)) != hipSuccess ||
-                hipMemcpy(g->d_nbr_p, pn, sizeof(int4) * (total > 0 ? total : 1), hipMemcpyHostToDevice) !=
-                    hipSuccess ||
-                hipMemcpy(g->d_nbs_p, ps, sizeof(float4) * (total > 0 ? total : 1), hipMemcpyHostToDevice) !=
-                    hipSuccess) {
-                free(pn);
-                free(ps);
-                return gerror_(engine_err_gpu, "neighbour list upload failed");
-            }
-            free(pn);
-            free(ps);
-        }
         free(cnt);
         free(fill);
         free(off);
@@ -2337,21 +2165,20 @@ extern "C" int engine_gpu_load(struct engine *e) {
     }
 
     /* Half-shell lists: the self task and each pair task once, at the task's
-       i cell, in task order; each cell's self entry; and for each cell the
-       pair entries that visit it as the task's j cell, in task order. */
+       i cell, in the order of the full-shell list; for each cell the i cells
+       that visit it as the task's j cell, in task order, each at slot
+       1 + its position (slot 0 is the self task), which the entry carries in
+       its bits 9 and up. */
     {
         const int nc = s->nr_cells;
         int *hcnt = (int *)calloc(nc + 1, sizeof(int)), *icnt = (int *)calloc(nc + 1, sizeof(int));
         int *hoff = (int *)malloc(sizeof(int) * (nc + 1)), *ioff = (int *)malloc(sizeof(int) * (nc + 1));
         int *hfill = (int *)malloc(sizeof(int) * (nc + 1)), *ifill = (int *)malloc(sizeof(int) * (nc + 1));
-        int *self_e = (int *)malloc(sizeof(int) * (nc > 0 ? nc : 1));
         int htot = 0, itot = 0, bad = 0;
         int4 *nbr = NULL;
         float4 *nbs = NULL;
-        int *ilist = NULL;
-        if (hcnt == NULL || icnt == NULL || hoff == NULL || ioff == NULL || hfill == NULL || ifill == NULL ||
-            self_e == NULL)
-            bad = 1;
+        int *icell = NULL;
+        if (hcnt == NULL || icnt == NULL || hoff == NULL || ioff == NULL || hfill == NULL || ifill == NULL) bad = 1;
         for (k = 0; !bad && k < s->nr_tasks; k++) {
             const struct task *t = &s->tasks[k];
             if (t->type == task_type_self)
@@ -2363,10 +2190,11 @@ extern "C" int engine_gpu_load(struct engine *e) {
         }
         if (!bad) {
             hoff[0] = ioff[0] = 0;
+            g->nslots = 1;
             for (cid = 0; cid < nc; cid++) {
                 hoff[cid + 1] = hoff[cid] + hcnt[cid];
                 ioff[cid + 1] = ioff[cid] + icnt[cid];
-                self_e[cid] = -1;
+                if (icnt[cid] + 1 > g->nslots) g->nslots = icnt[cid] + 1;
             }
             htot = hoff[nc];
             itot = ioff[nc];
@@ -2374,40 +2202,39 @@ extern "C" int engine_gpu_load(struct engine *e) {
             memcpy(ifill, ioff, sizeof(int) * (nc + 1));
             nbr = (int4 *)malloc(sizeof(int4) * (htot > 0 ? htot : 1));
             nbs = (float4 *)malloc(sizeof(float4) * (htot > 0 ? htot : 1));
-            ilist = (int *)malloc(sizeof(int) * (itot > 0 ? itot : 1));
-            if (nbr == NULL || nbs == NULL || ilist == NULL) bad = 1;
+            icell = (int *)malloc(sizeof(int) * (itot > 0 ? itot : 1));
+            if (nbr == NULL || nbs == NULL || icell == NULL) bad = 1;
         }
-        for (k = 0; !bad && k < s->nr_tasks; k++) {
-            const struct task *t = &s->tasks[k];
-            if (t->type == task_type_self) {
-                const int en = hfill[t->i]++;
-                self_e[t->i] = en;
-                nbs[en] = make_float4(0.f, 0.f, 0.f, 0.f);
-                nbr[en] = make_int4(t->i, 1 << 5, 0, 0);
-            } else if (t->type == task_type_pair) {
-                int dr, dp;
-                const int en = hfill[t->i]++;
-                task_dnshift(s, t->i, t->j, t->flags, g->P.dscale, &dr, &dp);
-                nbs[en] = cell_shift32(s, t->i, t->j);
-                nbr[en] = make_int4(t->j, t->flags, dr, dp);
-                ilist[ifill[t->j]++] = en;
+        /* entries without a window test first (win 0), then the others */
+        for (int win = 0; !bad && win < 2; win++)
+            for (k = 0; k < s->nr_tasks; k++) {
+                const struct task *t = &s->tasks[k];
+                if (t->type == task_type_self && win == 0) {
+                    const int en = hfill[t->i]++;
+                    nbs[en] = make_float4(0.f, 0.f, 0.f, 0.f);
+                    nbr[en] = make_int4(t->i, 1 << 5, 0, 0);
+                } else if (t->type == task_type_pair) {
+                    int dr, dp;
+                    task_dnshift(s, t->i, t->j, t->flags, g->P.dscale, &dr, &dp);
+                    if (task_window(g, s, dr, dp) != win) continue;
+                    const int en = hfill[t->i]++;
+                    const int slot = 1 + ifill[t->j] - ioff[t->j];
+                    nbs[en] = cell_shift32(s, t->i, t->j);
+                    nbr[en] = make_int4(t->j, t->flags | (win << 8) | (slot << 9), dr, dp);
+                    icell[ifill[t->j]++] = t->i;
+                }
             }
-        }
         if (!bad) {
-            g->n_entries_h = htot;
             if (hipMalloc(&g->d_nbr_h, sizeof(int4) * (htot > 0 ? htot : 1)) != hipSuccess ||
                 hipMalloc(&g->d_nbs_h, sizeof(float4) * (htot > 0 ? htot : 1)) != hipSuccess ||
                 hipMalloc(&g->d_nbr_off_h, sizeof(int) * (nc + 1)) != hipSuccess ||
-                hipMalloc(&g->d_self_entry, sizeof(int) * (nc > 0 ? nc : 1)) != hipSuccess ||
                 hipMalloc(&g->d_inv_off, sizeof(int) * (nc + 1)) != hipSuccess ||
-                hipMalloc(&g->d_inv_list, sizeof(int) * (itot > 0 ? itot : 1)) != hipSuccess ||
+                hipMalloc(&g->d_inv_cell, sizeof(int) * (itot > 0 ? itot : 1)) != hipSuccess ||
                 hipMemcpy(g->d_nbr_h, nbr, sizeof(int4) * (htot > 0 ? htot : 1), hipMemcpyHostToDevice) != hipSuccess ||
                 hipMemcpy(g->d_nbs_h, nbs, sizeof(float4) * (htot > 0 ? htot : 1), hipMemcpyHostToDevice) != hipSuccess ||
                 hipMemcpy(g->d_nbr_off_h, hoff, sizeof(int) * (nc + 1), hipMemcpyHostToDevice) != hipSuccess ||
-                hipMemcpy(g->d_self_entry, self_e, sizeof(int) * (nc > 0 ? nc : 1), hipMemcpyHostToDevice) !=
-                    hipSuccess ||
                 hipMemcpy(g->d_inv_off, ioff, sizeof(int) * (nc + 1), hipMemcpyHostToDevice) != hipSuccess ||
-                hipMemcpy(g->d_inv_list, ilist, sizeof(int) * (itot > 0 ? itot : 1), hipMemcpyHostToDevice) !=
+                hipMemcpy(g->d_inv_cell, icell, sizeof(int) * (itot > 0 ? itot : 1), hipMemcpyHostToDevice) !=
                     hipSuccess)
                 bad = 2;
         }
@@ -2417,10 +2244,9 @@ extern "C" int engine_gpu_load(struct engine *e) {
         free(ioff);
         free(hfill);
         free(ifill);
-        free(self_e);
         free(nbr);
         free(nbs);
-        free(ilist);
+        free(icell);
         if (bad) return gerror_(bad == 1 ? engine_err_malloc : engine_err_gpu, "half-shell lists");
     }
 
@@ -2500,7 +2326,21 @@ extern "C" int engine_gpu_load(struct engine *e) {
         g->nsplit = (MD_SPLIT_ITEMS_PER_CU * g->ncu + s->nr_cells - 1) / s->nr_cells;
         if (g->nsplit > MD_SPLIT_MAX) g->nsplit = MD_SPLIT_MAX;
     }
-    g->P.nsplit = g->nsplit;
+    /* k_pair: one wave per item, at most MD_PAIR_ITEMS_PER_CU items per CU,
+       whatever the cells hold (3 to 4 waves per SIMD are resident: with more
+       items a second turn of waves starts).  us at 8, 12, 16, 20 and 28 items
+       per CU: argon 1331 cells 66, 53, 52, 52, 60; mixture 125 cells 120, 114,
+       137, 136, 138, 729 cells 170, 122, 114, 134, 132; water 512 cells 408,
+       329, 414, 375, 395, 729 cells 706, 497, 575, 546, 574; and unsplit: argon
+       64 cells 82, now 30, mixture 125 cells 618, now 114. */
+    g->nsplit_t = 1;
+    if (!(e->flags & engine_flag_nosplit)) {
+        int cap = g->maxnbr / 2 < MD_PAIR_SPLIT_MAX ? g->maxnbr / 2 : MD_PAIR_SPLIT_MAX;
+        g->nsplit_t = MD_PAIR_ITEMS_PER_CU * g->ncu / s->nr_cells;
+        if (g->nsplit_t > cap) g->nsplit_t = cap;
+        if (g->nsplit_t < 1) g->nsplit_t = 1;
+    }
+    const int maxsplit = g->nsplit > g->nsplit_t ? g->nsplit : g->nsplit_t;
     {
         /* Owner cells in blocks of 6x6x6, blocks and the cells inside them in
            raster order: the owners a compute die works on at once, and their
@@ -2526,9 +2366,10 @@ extern "C" int engine_gpu_load(struct engine *e) {
         free(ord);
         g->P.order = g->d_order;
     }
+    HIPCHECK(hipMalloc(&g->d_kminmax, sizeof(unsigned short) * 26 * (size_t)s->nr_cells));
     HIPCHECK(hipMalloc(&g->d_cnt_off, sizeof(int2) * s->nr_cells));
-    HIPCHECK(hipMalloc(&g->d_cell_acc, sizeof(double) * 3 * (size_t)s->nr_cells * g->nsplit));
-    HIPCHECK(hipMalloc(&g->d_cell_cnt, sizeof(unsigned long long) * 3 * (size_t)s->nr_cells * g->nsplit));
+    HIPCHECK(hipMalloc(&g->d_cell_acc, sizeof(double) * 3 * (size_t)s->nr_cells * maxsplit));
+    HIPCHECK(hipMalloc(&g->d_cell_cnt, sizeof(unsigned long long) * 3 * (size_t)s->nr_cells * maxsplit));
     HIPCHECK(hipMalloc(&g->d_tot, sizeof(double) * 4));
     HIPCHECK(hipMalloc(&g->d_red_acc, sizeof(double) * 3 * MD_RED_BLOCKS));
     HIPCHECK(hipMalloc(&g->d_red_cnt, sizeof(unsigned long long) * 3 * MD_RED_BLOCKS));
@@ -2545,7 +2386,6 @@ extern "C" int engine_gpu_load(struct engine *e) {
     HIPCHECK(hipHostMalloc((void **)&g->h_tot, sizeof(double) * 4, hipHostMallocDefault));
     HIPCHECK(hipHostMalloc((void **)&g->h_tot_cnt, sizeof(unsigned long long) * 4, hipHostMallocDefault));
 
-    for (int k = 0; k < 8; k++) g->lds_nb[k] = 0;
     return engine_err_ok;
 }
 
@@ -2594,52 +2434,58 @@ int gpu_upload(struct engine *e) {
     return engine_err_ok;
 }
 
-/* Launch the kernels of one pass; optional events around each. */
-/* One device pass on the resident particles; mlp selects the surrogate
-   mode of the pair kernel. */
+/* Launch the kernels of one pass on the resident particles, with events
+   around each when timed; mlp selects the surrogate mode of the pair kernel.
+   sort: 0 keeps the keys and sort lists of the last sort. */
 int gpu_launch(struct gpu_state *g, int timed, int mlp, int sort) {
-    /* kernel: 0 table, 1 surrogate, 2 table with the 5-wave budget, 3 / 4
-       the half-shell table kernels (4 / 5 waves), 5 the half-shell
-       surrogate kernel, 6 / 7 the paired table kernels (4 / 5 waves; not
-       for the projected window, whose pass also counts the reference
-       window's pairs) */
-    const int wide = g->ncells >= 4 * 16 * g->ncu;
-    const int kern = mlp      ? (g->mlp_half ? 5 : 1)
-                     : g->half ? (wide ? 4 : 3)
-                     : (g->paired && !g->P.proj) ? (wide ? 7 : 6)
-                                 : (wide ? 2 : 0);
+    /* 32 owner atoms at a time while most cells fit (argon 108,000 atoms, at
+       26 and 32 per cell: 95 and 93 us against 135 and 131 with 64, whose LDS
+       share and registers leave 3 waves per SIMD instead of 4); beyond, the
+       cell's neighbours would be staged twice (at 39, 49 and 62 per cell 201,
+       226 and 213 us with 32, 135, 157 and 149 with 64; water at 125 per cell
+       434 and 328) */
+    const int big = (long long)g->nparts > (long long)MD_PAIR_R64_MEAN * g->ncells;
+    const int half = mlp ? g->mlp_half : g->half, pair = !mlp && !half;
+    /* table mode on the half shell: 5 waves per SIMD where the cells fill
+       them (measured equal to 4 at 64 cells per CU, ahead above) */
+    const int wide = !mlp && half && g->ncells >= 64 * g->ncu;
     struct nb_params P = g->P;
+    P.walk_cap = g->ncells >= 64 * g->ncu ? MD_HCAP_WIDE : MD_HCAP;
+    const int nsplit = P.nsplit = pair ? g->nsplit_t : g->nsplit;
     int nb;
     size_t lds = 0;
     const size_t maxn = (size_t)P.maxn;
-    lds = sizeof(float4) * 64; /* raw */
-    P.lds_own_key = (int)lds;
-    lds += sizeof(unsigned short) * 13 * 64;
-    lds = (lds + 15) & ~(size_t)15;
-    P.lds_kfl = (int)lds;
-    lds += sizeof(int) * 32;
-    lds = (lds + 15) & ~(size_t)15;
-    P.lds_stage = (int)lds;
-    lds += sizeof(float4) * maxn * (kern >= 6 ? 2 : 1); /* paired visits stage two cells */
-    P.lds_hit = (int)lds;
-    lds += sizeof(unsigned short) * 64 * (mlp ? MD_HCAP_MLP : (kern == 2 || kern == 7) ? MD_HCAP_WIDE : MD_HCAP);
-    lds = (lds + 15) & ~(size_t)15;
-    P.lds_dense = (int)lds;
-    if (mlp) lds += 16 * 64 * MD_HCAP_MLP + 4 * 64 * MD_XCAP_MLP + sizeof(float) * 2 * MLP_H;
-    lds = (lds + 15) & ~(size_t)15;
-    P.lds_jf = (int)lds;
-    if (kern >= 3 && kern <= 5) lds += sizeof(float) * 4 * 3 * maxn;
-    if (lds > 64 * 1024) return gerror_(engine_err_maxparts, "LDS staging exceeds 64 KiB");
-    if (kern >= 3 && kern <= 5 && (g->d_jpart == NULL || g->jcap < (int)maxn)) {
-        /* per half-shell entry, room for the visited cell's atoms; no
-           pending pass may still use the old buffer */
+    if (!pair) {
+        lds = sizeof(float4) * 64; /* raw */
+        P.lds_own_key = (int)lds;
+        lds += sizeof(unsigned short) * 13 * 64;
+        lds = (lds + 15) & ~(size_t)15;
+        P.lds_kfl = (int)lds;
+        lds += sizeof(int) * 32;
+        lds = (lds + 15) & ~(size_t)15;
+        P.lds_stage = (int)lds;
+        lds += sizeof(float4) * maxn;
+        P.lds_hit = (int)lds;
+        lds += sizeof(unsigned short) * 64 * (mlp ? MD_HCAP_MLP : wide ? MD_HCAP_WIDE : MD_HCAP);
+        lds = (lds + 15) & ~(size_t)15;
+        P.lds_dense = (int)lds;
+        if (mlp) lds += 16 * 64 * MD_HCAP_MLP + 4 * 64 * MD_XCAP_MLP + sizeof(float) * 2 * MLP_H;
+        lds = (lds + 15) & ~(size_t)15;
+        P.lds_jf = (int)lds;
+        if (half) lds += sizeof(float) * 4 * 3 * maxn;
+        if (lds > 64 * 1024) return gerror_(engine_err_maxparts, "LDS staging exceeds 64 KiB");
+    }
+    if (half && g->jcap < (size_t)g->nslots * g->nparts) {
+        /* per slot, the forces on every atom; no pending pass may still use
+           the old buffer */
         HIPCHECK(hipStreamSynchronize(g->stream));
         (void)hipFree(g->d_jpart);
         g->d_jpart = NULL;
-        g->jcap = (int)maxn + 8;
-        HIPCHECK(hipMalloc(&g->d_jpart, sizeof(float4) * (size_t)g->jcap * (g->n_entries_h > 0 ? g->n_entries_h : 1)));
+        g->jcap = 0;
+        HIPCHECK(hipMalloc(&g->d_jpart, sizeof(float) * 3 * (size_t)g->nslots * g->nparts));
+        g->jcap = (size_t)g->nslots * g->nparts;
     }
-    if (g->nsplit > 1 && g->pcap < (size_t)g->nsplit * g->nparts) {
+    if (nsplit > 1 && g->pcap < (size_t)nsplit * g->nparts) {
         /* per neighbour group, the owner forces of every atom; no pending
            pass may still use the old buffers */
         HIPCHECK(hipStreamSynchronize(g->stream));
@@ -2647,29 +2493,17 @@ int gpu_launch(struct gpu_state *g, int timed, int mlp, int sort) {
         (void)hipFree(g->d_plo);
         g->d_phi = g->d_plo = NULL;
         g->pcap = 0;
-        HIPCHECK(hipMalloc(&g->d_phi, sizeof(float4) * (size_t)g->nsplit * g->nparts));
-        HIPCHECK(hipMalloc(&g->d_plo, sizeof(float4) * (size_t)g->nsplit * g->nparts));
-        g->pcap = (size_t)g->nsplit * g->nparts;
+        HIPCHECK(hipMalloc(&g->d_phi, sizeof(float4) * (size_t)nsplit * g->nparts));
+        HIPCHECK(hipMalloc(&g->d_plo, sizeof(float4) * (size_t)nsplit * g->nparts));
+        g->pcap = (size_t)nsplit * g->nparts;
     }
-    if (lds != g->lds_nb[kern]) {
+    const int kern = mlp ? half : 2 + wide; /* kernels that walk the sorted windows */
+    if (!pair && lds != g->lds_nb[kern]) {
         /* Persistent grid: as many single-wave blocks as can be resident. */
+        const void *const fn[4] = {(const void *)k_nonbond_mlp, (const void *)k_nonbond_mlp_half,
+                                   (const void *)k_nonbond_half, (const void *)k_nonbond_half_wide};
         int per_cu = 0;
-        if (kern == 1)
-            HIPCHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_nonbond_mlp, 64, lds));
-        else if (kern == 5)
-            HIPCHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_nonbond_mlp_half, 64, lds));
-        else if (kern == 2)
-            HIPCHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_nonbond_wide, 64, lds));
-        else if (kern == 3)
-            HIPCHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_nonbond_half, 64, lds));
-        else if (kern == 4)
-            HIPCHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_nonbond_half_wide, 64, lds));
-        else if (kern == 6)
-            HIPCHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_nonbond_paired, 64, lds));
-        else if (kern == 7)
-            HIPCHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_nonbond_paired_wide, 64, lds));
-        else
-            HIPCHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_nonbond, 64, lds));
+        HIPCHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn[kern], 64, lds));
         if (per_cu < 1) per_cu = 1;
         g->grid_nb[kern] = g->ncu * per_cu;
         g->lds_nb[kern] = lds;
@@ -2684,8 +2518,8 @@ int gpu_launch(struct gpu_state *g, int timed, int mlp, int sort) {
     hipLaunchKernelGGL(k_pack, dim3(nb), dim3(256), 0, g->stream, g->nparts, g->d_x, g->d_type, g->d_id, g->ncells,
                        g->d_offset, g->d_xf, g->d_index_of_id, g->d_cell_of, g->d_queue);
     if (!sort) {
-        /* pseudo-Verlet step between rebuilds: the sort lists of the last
-           sort stay (runner.c:773) */
+        /* pseudo-Verlet step between rebuilds: the keys and sort lists of
+           the last sort stay (runner.c:773) */
     } else if (g->maxcount <= MD_SORT_LDS_MAX) {
         const int maxn = g->maxcount > 0 ? g->maxcount : 1;
         const size_t sh = sizeof(double) * 3 * maxn + sizeof(unsigned int) * 13 * maxn +
@@ -2694,11 +2528,12 @@ int gpu_launch(struct gpu_state *g, int timed, int mlp, int sort) {
            wave per direction */
         const int bs = maxn > MD_SORT_ONEWAVE_MAX ? 13 * 64 : 64;
         hipLaunchKernelGGL(k_sort_rank, dim3(g->ncells), dim3(bs), sh, g->stream, P, g->d_count, g->d_offset,
-                           g->d_sortflags, g->d_x, g->d_sortlist, g->d_keyof, g->d_queue + MD_NQUEUE, maxn);
+                           g->d_sortflags, g->d_x, g->d_sortlist, g->d_keyof, g->d_kminmax, g->d_queue + MD_NQUEUE,
+                           maxn);
     } else {
         nb = (g->ncells * 13 + 255) / 256;
         hipLaunchKernelGGL(k_sort, dim3(nb), dim3(256), 0, g->stream, P, g->d_count, g->d_offset, g->d_sortflags,
-                           g->d_x, g->d_sortlist, g->d_keyof, g->d_queue + MD_NQUEUE);
+                           g->d_x, g->d_sortlist, g->d_keyof, g->d_kminmax, g->d_queue + MD_NQUEUE);
     }
     if (sort) g->sort_valid = 1;
     if (timed) HIPCHECK(hipEventRecord(g->ev[1], g->stream));
@@ -2708,50 +2543,44 @@ int gpu_launch(struct gpu_state *g, int timed, int mlp, int sort) {
     O.cell_acc = g->d_cell_acc;
     O.cell_cnt = g->d_cell_cnt;
     O.jpart = g->d_jpart;
-    O.jcap = g->jcap;
     O.phi = g->d_phi;
     O.plo = g->d_plo;
-    /* no more waves than work items: the dispatcher then spreads them over
-       all compute units */
-    const int nitems = g->ncells * g->nsplit;
-    const int grid = g->grid_nb[kern] < nitems ? g->grid_nb[kern] : nitems;
-    if (kern == 3 || kern == 4) {
-        hipLaunchKernelGGL(kern == 4 ? k_nonbond_half_wide : k_nonbond_half, dim3(grid), dim3(64), lds,
-                           g->stream, P, g->d_cnt_off, g->d_nbr_h, g->d_nbr_off_h, g->d_nbs_h, g->d_origin, g->d_loc,
-                           g->d_xf, g->d_x, g->d_id, g->d_sortlist, g->d_keyof, g->d_ptab,
-                           (const float4 *)g->d_coeffs, g->d_excl_off, g->d_excl_list, g->d_index_of_id,
-                           g->d_cell_of, O, g->d_queue);
-    } else if (kern == 5)
-        hipLaunchKernelGGL(k_nonbond_mlp_half, dim3(grid), dim3(64), lds, g->stream, P, g->d_cnt_off, g->d_nbr_h,
-                           g->d_nbr_off_h, g->d_nbs_h, g->d_origin, g->d_loc, g->d_xf, g->d_x, g->d_id, g->d_sortlist,
-                           g->d_keyof, g->d_ptab, (const float4 *)g->d_coeffs, g->d_excl_off, g->d_excl_list,
-                           g->d_index_of_id, g->d_cell_of, O, g->d_queue, gpu_mlp_net(g), g->d_ptype);
-    else if (kern == 1)
-        hipLaunchKernelGGL(k_nonbond_mlp, dim3(grid), dim3(64), lds, g->stream, P, g->d_cnt_off, g->d_nbr,
-                           g->d_nbr_off, g->d_nbs, g->d_origin, g->d_loc, g->d_xf, g->d_x, g->d_id, g->d_sortlist,
-                           g->d_keyof, g->d_ptab, (const float4 *)g->d_coeffs, g->d_excl_off, g->d_excl_list,
-                           g->d_index_of_id, g->d_cell_of, O, g->d_queue, gpu_mlp_net(g), g->d_ptype);
-    else if (kern >= 6)
-        hipLaunchKernelGGL(kern == 7 ? k_nonbond_paired_wide : k_nonbond_paired, dim3(grid), dim3(64), lds, g->stream,
-                           P, g->d_cnt_off, g->d_nbr_p,
-                           g->d_nbr_off, g->d_nbs_p, g->d_origin, g->d_loc, g->d_xf, g->d_x, g->d_id, g->d_sortlist,
-                           g->d_keyof, g->d_ptab, (const float4 *)g->d_coeffs, g->d_excl_off, g->d_excl_list,
-                           g->d_index_of_id, g->d_cell_of, O, g->d_queue);
-    else
-        hipLaunchKernelGGL(kern == 2 ? k_nonbond_wide : k_nonbond, dim3(grid), dim3(64), lds, g->stream,
-                           P, g->d_cnt_off, g->d_nbr,
-                           g->d_nbr_off, g->d_nbs, g->d_origin, g->d_loc, g->d_xf, g->d_x, g->d_id, g->d_sortlist,
-                           g->d_keyof, g->d_ptab, (const float4 *)g->d_coeffs, g->d_excl_off, g->d_excl_list,
-                           g->d_index_of_id, g->d_cell_of, O, g->d_queue);
-    if ((kern >= 3 && kern <= 5) || g->nsplit > 1)
-        hipLaunchKernelGGL(k_fold, dim3(g->ncells), dim3(64), 0, g->stream, g->ncells, g->d_cnt_off, g->nsplit,
-                           g->nparts, (const float4 *)g->d_phi, (const float4 *)g->d_plo,
-                           (kern >= 3 && kern <= 5) ? 1 : 0,
-                           g->d_self_entry, g->d_inv_off, g->d_inv_list, (const float4 *)g->d_jpart, g->jcap,
-                           g->d_fhi, g->d_flo);
+    const int nitems = g->ncells * nsplit;
+    if (pair) {
+        static const decltype(&k_pair<32, false>) kp[2][2] = {{k_pair<32, false>, k_pair<32, true>},
+                                                              {k_pair<64, false>, k_pair<64, true>}};
+        /* the same number of blocks for each die */
+        const dim3 grid((nitems + MD_NQUEUE - 1) / MD_NQUEUE * MD_NQUEUE);
+        hipLaunchKernelGGL(kp[big][P.proj != 0], grid, dim3(64), 0, g->stream, P, g->d_cnt_off, g->d_nbr, g->d_nbr_off,
+                           g->d_nbr_mid, g->d_nbs, g->d_origin, g->d_loc, g->d_xf, g->d_x, g->d_id,
+                           g->d_kminmax, g->d_sortlist, g->d_keyof, g->d_ptab, (const float4 *)g->d_coeffs,
+                           g->d_excl_off, g->d_excl_list, g->d_index_of_id, g->d_cell_of, O);
+    } else {
+        /* no more waves than work items: the dispatcher then spreads them
+           over all compute units */
+        const dim3 grid(g->grid_nb[kern] < nitems ? g->grid_nb[kern] : nitems);
+        const int4 *nbr = half ? g->d_nbr_h : g->d_nbr;
+        const int *off = half ? g->d_nbr_off_h : g->d_nbr_off;
+        const float4 *nbs = half ? g->d_nbs_h : g->d_nbs;
+        if (mlp)
+            hipLaunchKernelGGL(half ? k_nonbond_mlp_half : k_nonbond_mlp, grid, dim3(64), lds, g->stream, P,
+                               g->d_cnt_off, nbr, off, nbs, g->d_origin, g->d_loc, g->d_xf, g->d_x, g->d_id,
+                               g->d_sortlist, g->d_keyof, g->d_ptab, (const float4 *)g->d_coeffs, g->d_excl_off,
+                               g->d_excl_list, g->d_index_of_id, g->d_cell_of, O, g->d_queue, gpu_mlp_net(g),
+                               g->d_ptype);
+        else
+            hipLaunchKernelGGL(wide ? k_nonbond_half_wide : k_nonbond_half, grid, dim3(64), lds, g->stream, P,
+                               g->d_cnt_off, nbr, off, nbs, g->d_origin, g->d_loc, g->d_xf, g->d_x, g->d_id,
+                               g->d_sortlist, g->d_keyof, g->d_ptab, (const float4 *)g->d_coeffs, g->d_excl_off,
+                               g->d_excl_list, g->d_index_of_id, g->d_cell_of, O, g->d_queue);
+    }
+    if (half || nsplit > 1)
+        hipLaunchKernelGGL(k_fold, dim3(g->ncells), dim3(64), 0, g->stream, g->ncells, g->d_cnt_off, nsplit,
+                           g->nparts, (const float4 *)g->d_phi, (const float4 *)g->d_plo, half,
+                           g->d_inv_off, g->d_inv_cell, g->d_jpart, g->d_fhi, g->d_flo);
     if (timed) HIPCHECK(hipEventRecord(g->ev[2], g->stream));
-    hipLaunchKernelGGL(k_reduce_a, dim3(MD_RED_BLOCKS), dim3(256), 0, g->stream, g->ncells * g->nsplit,
-                       g->d_cell_acc, g->d_cell_cnt, g->d_red_acc, g->d_red_cnt);
+    hipLaunchKernelGGL(k_reduce_a, dim3(MD_RED_BLOCKS), dim3(256), 0, g->stream, nitems, g->d_cell_acc, g->d_cell_cnt,
+                       g->d_red_acc, g->d_red_cnt);
     hipLaunchKernelGGL(k_reduce_b, dim3(1), dim3(256), 0, g->stream, MD_RED_BLOCKS, g->d_red_acc, g->d_red_cnt,
                        g->d_tot, g->d_tot_cnt);
     if (timed) HIPCHECK(hipEventRecord(g->ev[3], g->stream));

@@ -44,11 +44,14 @@ struct nb_params {
     int lds_own_key, lds_kfl, lds_stage, lds_hit, lds_dense, lds_jf;
     int nsplit; /* neighbour groups per owner cell (work items per cell) */
     const int *order; /* owner cell of each owner position in the work order */
+    int window; /* some entries need the reference's window test (pair_tile.h) */
+    float filt; /* k_pair's filter threshold on r^2 */
+    int walk_cap; /* k_pair, projected window: see pair_tile.h */
 };
 
 /* Neighbour-list entry of an owner cell: x = other cell, y = sid | orient<<4
-   | self<<5 (orient 0: owner is the task's i cell), z = dnshift with the
-   reference window |shift|, w = dnshift with the projected shift.n.
+   | self<<5 | window<<8 (orient 0: owner is the task's i cell; window: see
+   pair_tile.h; half shell: jpart slot<<9, else distance class<<16), z = dnshift with the reference window |shift|, w = dnshift with the projected shift.n.
    Type-pair table header ptab[ti*mt+tj] = (alpha0, alpha1, alpha2,
    bits(n | chunk0 << 9)) or w = bits(-1) when the pair has no potential. */
 
@@ -60,35 +63,29 @@ struct gpu_state {
     int maxcell; /* particles per cell the packed record holds */
     int nparts, nids;
     struct nb_params P;
-    /* [0] table mode, [1] surrogate mode, [2] table mode with the 5-wave
-       budget, [3] / [4] the half-shell table kernels with 4 / 5 waves, [5]
-       the half-shell surrogate kernel, [6] / [7] the paired table kernels
-       with 4 / 5 waves */
-    int grid_nb[8], ncu;
-    size_t lds_nb[8];
+    /* persistent grid and dynamic LDS of the kernels that walk the sorted
+       windows: surrogate full and half shell, table half shell, its 5-wave build */
+    int grid_nb[4], ncu;
+    size_t lds_nb[4];
     /* static */
     float4 *d_ptab;
     float *d_coeffs;
     int4 *d_nbr;
     float4 *d_nbs; /* per neighbour entry: FP32 minimum-image shift owner -> neighbour */
-    int *d_nbr_off;
-    /* the same entries with those of opposite offsets side by side: the
-       first of a pair (its owner is the task's i cell) has bit 6 of .y set,
-       its partner bit 7 */
-    int4 *d_nbr_p;
-    float4 *d_nbs_p;
+    int *d_nbr_off, *d_nbr_mid; /* d_nbr: i side first; its j side from mid */
     int paired; /* set unless engine_flag_unpaired */
-    /* half shell: each task once at its i cell; the self entry of each cell;
-       the entries that visit each cell as a task's j cell; per entry the
-       forces on the visited atoms (jcap slots) */
+    /* half shell: each task once at its i cell; the i cells that visit each
+       cell as a task's j cell; per slot (0: self task, 1..: those visits) the
+       forces on every atom (jcap atoms in all) */
     int4 *d_nbr_h;
     float4 *d_nbs_h;
-    int *d_nbr_off_h, *d_self_entry, *d_inv_off, *d_inv_list;
-    int n_entries_h, jcap, half, mlp_half;
-    float4 *d_jpart;
+    int *d_nbr_off_h, *d_inv_off, *d_inv_cell;
+    int nslots, half, mlp_half;
+    size_t jcap;
+    float *d_jpart;
     /* split owners: nsplit neighbour groups per cell; per group the owner
        forces of every atom (pcap float4 allocated in each) */
-    int nsplit;
+    int nsplit, nsplit_t; /* kernels that walk the sorted windows; k_pair */
     size_t pcap;
     float4 *d_phi, *d_plo;
     double *d_origin;
@@ -103,6 +100,7 @@ struct gpu_state {
     float4 *d_xf, *d_fhi, *d_flo;
     unsigned int *d_sortlist;
     unsigned short *d_keyof;
+    unsigned short *d_kminmax; /* per cell: largest key of the 13 directions, then the smallest */
     double *d_cell_acc, *d_tot;
     unsigned long long *d_cell_cnt, *d_tot_cnt;
     double *d_red_acc; /* per-block partial sums of the totals */
@@ -164,8 +162,8 @@ void gpu_mlp_free(struct gpu_state *g);
 void gpu_steps_free(struct gpu_state *g);
 
 /* engine_gpu.hip: pack the host cells and upload them (no kernels); launch
-   one pass on the resident particles (mlp: surrogate mode; sort == 0 keeps
-   the sort lists of the last sort), with events around each kernel when
+   one pass on the resident particles (mlp: surrogate mode; sort: 0 keeps the
+   keys and sort lists of the last sort), with events around each kernel when
    timed. */
 int gpu_upload(struct engine *e);
 int gpu_launch(struct gpu_state *g, int timed, int mlp, int sort);
