@@ -38,7 +38,8 @@
  *               hits evaluated with the network;
  *   k_fold      per atom, the groups' partial forces and the half-shell
  *               slots, added in a fixed order;
- *   k_reduce_a/b per-item FP64 energies/virials/counts -> totals, fixed order.
+ *   k_reduce_one (few items) or k_reduce_a/b
+ *               per-item FP64 energies/virials/counts -> totals, fixed order.
  * Staged neighbour records hold their positions moved into the owner's
  * frame (x + shift, once per record), so a candidate's distance is one
  * subtraction per axis.  In the full shell every pair is evaluated by both
@@ -716,14 +717,20 @@ __device__ void sort_lists_wave(unsigned int *a, int n, unsigned int tm, unsigne
    included, so those particles are placed by counting.  Only the order of
    equal keys depends on the quicksort's partitions: a list with equal keys
    is sorted again with the reference's algorithm (runner.c:110-174), in LDS,
-   and written whole.  Cells of at most MD_SORT_ONEWAVE_MAX particles get one
-   wave, which sorts all such lists of its cell together (sort_lists_wave);
-   larger cells get 13 waves, wave l sorting list l (sort_desc_wave).  For
+   and written whole.  Cells of at most MD_SORT_ONEWAVE_MAX particles, more
+   than MD_SORT_FEW of them, get one wave, which sorts all such lists of its cell together (sort_lists_wave);
+   larger or few cells get 13 waves, wave l sorting list l (sort_desc_wave).  For
    cells of at most MD_SORT_LDS_MAX particles.  LDS: 3 * maxn positions,
    13 * maxn list words, 13 quicksort stacks, 13 pairs of partition tables
    and 136 more entries (the one-wave sort keeps its segment queues there). */
 #define MD_SORT_LDS_MAX 480 /* 63.5 KiB of LDS at 480 */
 #define MD_SORT_ONEWAVE_MAX 64
+/* Cells up to which every cell gets 13 waves: a cell's sorts are one serial
+   chain, which 13 waves shorten while the device has room for them.  us with
+   one wave and with 13: argon 64 cells 37, 27; 125 cells 34, 29 (mixture, with
+   more equal keys, 50, 33); 512 cells 36, 33; 1331 cells 37, 45; 10648 cells
+   69, 177. */
+#define MD_SORT_FEW 768
 __global__ __launch_bounds__(1024) void k_sort_rank(struct nb_params P, const int *__restrict__ count,
                                                   const int *__restrict__ offset,
                                                   const unsigned int *__restrict__ sortflags,
@@ -742,11 +749,12 @@ __global__ __launch_bounds__(1024) void k_sort_rank(struct nb_params P, const in
     if (n == 0) return;
     const unsigned int fl = sortflags[c];
     const int off = offset[c];
+    const float rn = 1.0f / (float)n;
     if (lane < 13) tie[lane] = 0;
     for (int k = lane; k < 3 * n; k += (int)blockDim.x) xs[k] = x[3 * (size_t)off + k];
     __syncthreads();
     for (int t = lane; t < 13 * n; t += (int)blockDim.x) {
-        const int sid = t / n, i = t - sid * n;
+        const int sid = (int)(((float)t + 0.5f) * rn), i = t - sid * n; /* t / n */
         if (!((fl >> sid) & 1u)) continue;
         const unsigned int key = sort_key(&xs[3 * i], sid, P.dscale, P.bias);
         lists[sid * n + i] = ((unsigned int)i << 16) | key;
@@ -755,7 +763,7 @@ __global__ __launch_bounds__(1024) void k_sort_rank(struct nb_params P, const in
     __syncthreads();
     unsigned int *out = sortlist + 13 * (size_t)off;
     for (int t = lane; t < 13 * n; t += (int)blockDim.x) {
-        const int sid = t / n, i = t - sid * n;
+        const int sid = (int)(((float)t + 0.5f) * rn), i = t - sid * n; /* t / n */
         if (!((fl >> sid) & 1u)) continue;
         const unsigned int *L = lists + sid * n;
         const unsigned int w = L[i], key = w & 0xffffu;
@@ -1668,6 +1676,41 @@ __device__ __forceinline__ void block_tree3(double (*sd)[256], unsigned long lon
     }
 }
 
+/* The totals of few items in one launch, by one block: 4.4 us at 3,000 items
+   against 8 us and another launch for the two above; a block's 256 threads
+   load 32 items each at MD_RED_ONE. */
+#define MD_RED_ONE 8192
+__global__ __launch_bounds__(256) void k_reduce_one(int n, const double *__restrict__ acc,
+                                                    const unsigned long long *__restrict__ cnt,
+                                                    double *__restrict__ tot,
+                                                    unsigned long long *__restrict__ tot_cnt) {
+    __shared__ double sd[3][256];
+    __shared__ unsigned long long sc[3][256];
+    const int t = threadIdx.x;
+    double d0 = 0, d1 = 0, d2 = 0;
+    unsigned long long c0 = 0, c1 = 0, c2 = 0;
+#pragma unroll 4
+    for (int k = t; k < n; k += 256) {
+        d0 += acc[3 * k];
+        d1 += acc[3 * k + 1];
+        d2 += acc[3 * k + 2];
+        c0 += cnt[3 * k];
+        c1 += cnt[3 * k + 1];
+        c2 += cnt[3 * k + 2];
+    }
+    sd[0][t] = d0;
+    sd[1][t] = d1;
+    sd[2][t] = d2;
+    sc[0][t] = c0;
+    sc[1][t] = c1;
+    sc[2][t] = c2;
+    block_tree3(sd, sc, t);
+    if (t < 3) {
+        tot[t] = sd[t][0];
+        tot_cnt[t] = sc[t][0];
+    }
+}
+
 __global__ __launch_bounds__(256) void k_reduce_a(int n, const double *__restrict__ acc,
                                                   const unsigned long long *__restrict__ cnt,
                                                   double *__restrict__ pacc, unsigned long long *__restrict__ pcnt) {
@@ -2524,9 +2567,9 @@ int gpu_launch(struct gpu_state *g, int timed, int mlp, int sort) {
         const int maxn = g->maxcount > 0 ? g->maxcount : 1;
         const size_t sh = sizeof(double) * 3 * maxn + sizeof(unsigned int) * 13 * maxn +
                           sizeof(int) * 13 * 2 * MD_SORT_STACK + sizeof(unsigned short) * (13 * 2 * (maxn + 1) + 136);
-        /* one wave per cell; for large cells (frequent repeated keys) one
-           wave per direction */
-        const int bs = maxn > MD_SORT_ONEWAVE_MAX ? 13 * 64 : 64;
+        /* one wave per cell; for large cells (frequent repeated keys) and for
+           few cells one wave per direction */
+        const int bs = maxn > MD_SORT_ONEWAVE_MAX || g->ncells <= MD_SORT_FEW ? 13 * 64 : 64;
         hipLaunchKernelGGL(k_sort_rank, dim3(g->ncells), dim3(bs), sh, g->stream, P, g->d_count, g->d_offset,
                            g->d_sortflags, g->d_x, g->d_sortlist, g->d_keyof, g->d_kminmax, g->d_queue + MD_NQUEUE,
                            maxn);
@@ -2579,10 +2622,15 @@ int gpu_launch(struct gpu_state *g, int timed, int mlp, int sort) {
                            g->nparts, (const float4 *)g->d_phi, (const float4 *)g->d_plo, half,
                            g->d_inv_off, g->d_inv_cell, g->d_jpart, g->d_fhi, g->d_flo);
     if (timed) HIPCHECK(hipEventRecord(g->ev[2], g->stream));
-    hipLaunchKernelGGL(k_reduce_a, dim3(MD_RED_BLOCKS), dim3(256), 0, g->stream, nitems, g->d_cell_acc, g->d_cell_cnt,
-                       g->d_red_acc, g->d_red_cnt);
-    hipLaunchKernelGGL(k_reduce_b, dim3(1), dim3(256), 0, g->stream, MD_RED_BLOCKS, g->d_red_acc, g->d_red_cnt,
-                       g->d_tot, g->d_tot_cnt);
+    if (nitems <= MD_RED_ONE)
+        hipLaunchKernelGGL(k_reduce_one, dim3(1), dim3(256), 0, g->stream, nitems, g->d_cell_acc, g->d_cell_cnt,
+                           g->d_tot, g->d_tot_cnt);
+    else {
+        hipLaunchKernelGGL(k_reduce_a, dim3(MD_RED_BLOCKS), dim3(256), 0, g->stream, nitems, g->d_cell_acc,
+                           g->d_cell_cnt, g->d_red_acc, g->d_red_cnt);
+        hipLaunchKernelGGL(k_reduce_b, dim3(1), dim3(256), 0, g->stream, MD_RED_BLOCKS, g->d_red_acc, g->d_red_cnt,
+                           g->d_tot, g->d_tot_cnt);
+    }
     if (timed) HIPCHECK(hipEventRecord(g->ev[3], g->stream));
     HIPCHECK(hipGetLastError());
     return engine_err_ok;
