@@ -723,8 +723,6 @@ __device__ void sort_lists_wave(unsigned int *a, int n, unsigned int tm, unsigne
    cells of at most MD_SORT_LDS_MAX particles.  LDS: 3 * maxn positions,
    13 * maxn list words, 13 quicksort stacks, 13 pairs of partition tables
    and 136 more entries (the one-wave sort keeps its segment queues there). */
-#define MD_SORT_LDS_MAX 480 /* 63.5 KiB of LDS at 480 */
-#define MD_SORT_ONEWAVE_MAX 64
 /* Cells up to which every cell gets 13 waves: a cell's sorts are one serial
    chain, which 13 waves shorten while the device has room for them.  us with
    one wave and with 13: argon 64 cells 37, 27; 125 cells 34, 29 (mixture, with
@@ -746,7 +744,7 @@ __global__ __launch_bounds__(1024) void k_sort_rank(struct nb_params P, const in
     __shared__ int tie[13];
     const int c = blockIdx.x, lane = threadIdx.x;
     const int n = count[c];
-    if (n == 0) return;
+    if (n == 0 || n > maxn) return; /* a cell that outgrew the launch: the caller repeats it */
     const unsigned int fl = sortflags[c];
     const int off = offset[c];
     const float rn = 1.0f / (float)n;
@@ -2477,10 +2475,19 @@ int gpu_upload(struct engine *e) {
     return engine_err_ok;
 }
 
+/* No slot for any particle id. */
+int gpu_clear_ids(struct gpu_state *g) {
+    const int nb = (g->nids + 255) / 256;
+    if (nb > 0) hipLaunchKernelGGL(k_clear_ids, dim3(nb), dim3(256), 0, g->stream, g->nids, g->d_index_of_id);
+    HIPCHECK(hipGetLastError());
+    return engine_err_ok;
+}
+
 /* Launch the kernels of one pass on the resident particles, with events
    around each when timed; mlp selects the surrogate mode of the pair kernel.
-   sort: 0 keeps the keys and sort lists of the last sort. */
-int gpu_launch(struct gpu_state *g, int timed, int mlp, int sort) {
+   sort: 0 keeps the keys and sort lists of the last sort; packed: d_xf and
+   the id and cell maps are those of the particles already. */
+int gpu_launch(struct gpu_state *g, int timed, int mlp, int sort, int packed) {
     /* 32 owner atoms at a time while most cells fit (argon 108,000 atoms, at
        26 and 32 per cell: 95 and 93 us against 135 and 131 with 64, whose LDS
        share and registers leave 3 waves per SIMD instead of 4); beyond, the
@@ -2555,10 +2562,10 @@ int gpu_launch(struct gpu_state *g, int timed, int mlp, int sort) {
     if (!sort && !g->sort_valid) return gerror_(engine_err_range, "no sort lists to reuse");
 
     if (timed) HIPCHECK(hipEventRecord(g->ev[0], g->stream));
-    nb = (g->nids + 255) / 256;
-    if (nb > 0) hipLaunchKernelGGL(k_clear_ids, dim3(nb), dim3(256), 0, g->stream, g->nids, g->d_index_of_id);
+    if (!packed && gpu_clear_ids(g) < 0) return engine_err_gpu;
     nb = ((g->nparts > g->ncells ? g->nparts : g->ncells) + 255) / 256;
-    hipLaunchKernelGGL(k_pack, dim3(nb), dim3(256), 0, g->stream, g->nparts, g->d_x, g->d_type, g->d_id, g->ncells,
+    if (!packed)
+        hipLaunchKernelGGL(k_pack, dim3(nb), dim3(256), 0, g->stream, g->nparts, g->d_x, g->d_type, g->d_id, g->ncells,
                        g->d_offset, g->d_xf, g->d_index_of_id, g->d_cell_of, g->d_queue);
     if (!sort) {
         /* pseudo-Verlet step between rebuilds: the keys and sort lists of
@@ -2730,7 +2737,7 @@ extern "C" int engine_nonbond_gpu(struct engine *e) {
     int sort = 1;
     if (gpu_verlet(e, g, &sort) < 0) return engine_err_range;
     HIPCHECK(hipMemsetAsync(g->d_queue + MD_NQUEUE, 0, sizeof(int), g->stream));
-    if (gpu_launch(g, 1, (e->flags & engine_flag_mlp) != 0, sort) < 0) return engine_err_gpu;
+    if (gpu_launch(g, 1, (e->flags & engine_flag_mlp) != 0, sort, 0) < 0) return engine_err_gpu;
     if (sort) gpu_sorted(e, g);
     HIPCHECK(hipMemcpyAsync(g->h_fhi, g->d_fhi, sizeof(float4) * g->nparts, hipMemcpyDeviceToHost, g->stream));
     HIPCHECK(hipMemcpyAsync(g->h_flo, g->d_flo, sizeof(float4) * g->nparts, hipMemcpyDeviceToHost, g->stream));
@@ -2769,10 +2776,10 @@ extern "C" int engine_gpu_time(struct engine *e, int nsteps, int nwarm, double *
     /* the sort of a pass that engine_step would make, on the resident data */
     const int sort = !(e->flags & engine_flag_verlet) || e->s.verlet_rebuild || !g->sort_valid;
     for (k = 0; k < nwarm; k++)
-        if (gpu_launch(g, 0, (e->flags & engine_flag_mlp) != 0, sort) < 0) return engine_err_gpu;
+        if (gpu_launch(g, 0, (e->flags & engine_flag_mlp) != 0, sort, 0) < 0) return engine_err_gpu;
     HIPCHECK(hipStreamSynchronize(g->stream));
     for (k = 0; k < nsteps; k++) {
-        if (gpu_launch(g, 1, (e->flags & engine_flag_mlp) != 0, sort) < 0) return engine_err_gpu;
+        if (gpu_launch(g, 1, (e->flags & engine_flag_mlp) != 0, sort, 0) < 0) return engine_err_gpu;
         HIPCHECK(hipEventSynchronize(g->ev[3]));
         HIPCHECK(hipEventElapsedTime(&t, g->ev[0], g->ev[1]));
         acc[0] += t;

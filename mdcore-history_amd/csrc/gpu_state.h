@@ -14,6 +14,9 @@
 #define MD_MAX_CELL 1024  /* particles per cell: the packed record's slot field is 10 bits at most */
 #define MD_MAX_TYPES 1024 /* particle types: 6, 8 or 10 type bits, leaving 10, 8 or 6 slot bits */
 
+#define MD_SORT_LDS_MAX 480    /* k_sort_rank's cells: 63.5 KiB of LDS at 480 */
+#define MD_SORT_ONEWAVE_MAX 64 /* those of them that one wave sorts */
+
 #define gerror_(id, msg) errs_register((id), (msg), __LINE__, __func__, __FILE__)
 
 #define HIPCHECK(call)                                                                            \
@@ -163,10 +166,12 @@ void gpu_steps_free(struct gpu_state *g);
 
 /* engine_gpu.hip: pack the host cells and upload them (no kernels); launch
    one pass on the resident particles (mlp: surrogate mode; sort: 0 keeps the
-   keys and sort lists of the last sort), with events around each kernel when
-   timed. */
+   keys and sort lists of the last sort; packed: the FP32 positions and the id
+   and cell maps are the particles' already), with events around each kernel
+   when timed; clear the id map. */
 int gpu_upload(struct engine *e);
-int gpu_launch(struct gpu_state *g, int timed, int mlp, int sort);
+int gpu_launch(struct gpu_state *g, int timed, int mlp, int sort, int packed);
+int gpu_clear_ids(struct gpu_state *g);
 
 #endif /* GPU_STATE_H */
 

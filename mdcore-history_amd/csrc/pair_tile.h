@@ -241,7 +241,7 @@ __device__ __forceinline__ void pair_body(pair_lds<R> &L, const struct nb_params
                 eself = (en.y >> 5) & 1;
                 esid = en.y & 15;
                 eoff = co.y;
-                ecnt = co.x;
+                ecnt = min(co.x, MD_MAX_CELL); /* more fit no field; their pass is not used */
                 ewin = (en.y >> 8) & 1;
                 bool live = ecnt > 0;
                 if (!eself && ecnt > 0) {

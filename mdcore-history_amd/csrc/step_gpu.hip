@@ -5,20 +5,22 @@
  * engine_advance 1945-2052 and space_shuffle_local), with the particles kept
  * on the GPU between steps:
  *   1. shuffle: particles outside their cell move to the neighbour cell;
- *   2. the nonbonded pass (k_pack, k_sort*, k_nonbond*, k_reduce);
+ *   2. the nonbonded pass (k_sort*, the pair kernel, k_reduce*; its FP32
+ *      positions and maps come from the migration before it);
  *   3. kick-drift v += f dt / m, x += dt v in FP64, then migration.
  * Migration keeps the host's order exactly, so the sorted lists, the pair
  * sets and the trajectory are bitwise those of the host-driven loop:
  *   - per source cell, in storage order, a leaving particle is appended to
  *     its departures and the cell's last particle takes its slot (k_migrate,
  *     one wave per cell, with the kick fused in);
- *   - new counts and offsets come from a fixed-order three-pass scan
- *     (k_scan_a/b/c), arrival counts from atomic increments (a sum, so the
+ *   - new counts and offsets come from a fixed-order scan (k_scan_one, or
+ *     k_scan_a/b/c in three passes), arrival counts from atomic increments (a sum, so the
  *     order of the increments does not matter);
- *   - stayers keep their relative order (k_stayers); each destination
- *     appends its arrivals by source cell and departure order (k_arrive).
+ *   - stayers keep their relative order, and each destination appends
+ *     its arrivals by source cell and departure order (k_settle).
  * The host's shuffle at the start of a step moves nothing when the previous
- * advance left every particle inside its cell; it is then skipped.
+ * advance left every particle inside its cell; it is then skipped.  The next
+ * pass is launched before the host knows whether that is so (steps_ahead).
  * No reference counterpart as a device path: the reference's CUDA engine
  * returns to the host every step (runner_cuda.cu:2405-2430, 2514-2521).
  */
@@ -63,8 +65,8 @@ __global__ __launch_bounds__(64) void k_migrate(struct step_geom G, int kick, do
                                                 const float4 *__restrict__ fhi, const float4 *__restrict__ flo,
                                                 const int *__restrict__ count, const int *__restrict__ offset,
                                                 double *__restrict__ x, double *__restrict__ v,
-                                                const int *__restrict__ type, int *__restrict__ cell_of,
-                                                int *__restrict__ slot, int *__restrict__ qsrc,
+                                                const int *__restrict__ type, int *__restrict__ slot,
+                                                int *__restrict__ qsrc,
                                                 int *__restrict__ qdest, int *__restrict__ stay,
                                                 int *__restrict__ ndep, int *__restrict__ narr,
                                                 double *__restrict__ cell_ke) {
@@ -95,7 +97,6 @@ __global__ __launch_bounds__(64) void k_migrate(struct step_geom G, int kick, do
             ke += 0.5 * mass[t] * (vv[0] * vv[0] + vv[1] * vv[1] + vv[2] * vv[2]);
         }
         code[k] = (unsigned char)leave_code(xa, G.h);
-        cell_of[a] = c;
     }
     __syncthreads();
     if (lane == 0) {
@@ -237,24 +238,81 @@ __global__ __launch_bounds__(256) void k_scan_c(int ncells, const int *__restric
         }
 }
 
-/* Stayers: old slot a to its slot in the new layout. */
-__global__ __launch_bounds__(256) void k_stayers(int n, const int *__restrict__ cell_of, const int *__restrict__ slot,
-                                                 const int *__restrict__ new_off, const double *__restrict__ x,
-                                                 const double *__restrict__ v, const int *__restrict__ id,
-                                                 const int *__restrict__ type, double *__restrict__ x2,
-                                                 double *__restrict__ v2, int *__restrict__ id2,
-                                                 int *__restrict__ type2) {
-    const int a = blockIdx.x * blockDim.x + threadIdx.x;
-    if (a >= n) return;
-    const int r = slot[a];
-    if (r < 0) return;
-    const int b = new_off[cell_of[a]] + r;
-    for (int m = 0; m < 3; m++) {
-        x2[3 * b + m] = x[3 * a + m];
-        v2[3 * b + m] = v[3 * a + m];
+/* The three passes in one launch, by one block, for few cells: the same sums
+   in the same order.  Each round takes 4 blocks' cells: one round 5 us
+   against 12 us and two more launches, but 13,824 cells 25 us against 15. */
+#define MD_SCAN_ONE 4096
+__global__ __launch_bounds__(1024) void k_scan_one(int ncells, const int *__restrict__ stay, int *__restrict__ narr,
+                                                   const double *__restrict__ cell_ke, int *__restrict__ count,
+                                                   int *__restrict__ offset, int2 *__restrict__ cnt_off,
+                                                   int *__restrict__ st, const double *__restrict__ tot,
+                                                   double *__restrict__ esteps) {
+    __shared__ int ws[16], wm[16];
+    __shared__ double sk[1024];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    int base = 0, mx = 0;
+    double ke = 0.0;
+    for (int r0 = 0; r0 < ncells; r0 += 4 * MD_SCAN_CELLS) {
+        const int c0 = r0 + 4 * t;
+        int n[4] = {0, 0, 0, 0}, sum = 0;
+        double k4 = 0.0;
+        for (int k = 0; k < 4; k++)
+            if (c0 + k < ncells) {
+                n[k] = stay[c0 + k] + narr[c0 + k];
+                sum += n[k];
+                mx = n[k] > mx ? n[k] : mx;
+                if (cell_ke) k4 += cell_ke[c0 + k];
+            }
+        int run = sum;
+        for (int o = 1; o < 64; o <<= 1) {
+            const int v = __shfl_up(run, o);
+            if (lane >= o) run += v;
+        }
+        sk[t] = k4;
+        __syncthreads();
+        if (lane == 63) ws[w] = run;
+        __syncthreads();
+        int before = base, all = 0;
+        for (int k = 0; k < 16; k++) {
+            before += k < w ? ws[k] : 0;
+            all += ws[k];
+        }
+        run += before - sum;
+        for (int k = 0; k < 4; k++)
+            if (c0 + k < ncells) {
+                count[c0 + k] = n[k];
+                offset[c0 + k] = run;
+                cnt_off[c0 + k] = make_int2(n[k], run);
+                narr[c0 + k] = 0;
+                run += n[k];
+            }
+        base += all;
+        /* the kinetic energy as k_scan_a and k_scan_b add it */
+        for (int o = 128; o > 0; o >>= 1) {
+            if ((t & 255) < o) sk[t] += sk[t + o];
+            __syncthreads();
+        }
+        for (int b = 0; b < 4 && r0 + b * MD_SCAN_CELLS < ncells; b++) ke += sk[256 * b];
+        __syncthreads();
     }
-    id2[b] = id[a];
-    type2[b] = type[a];
+    for (int o = 32; o > 0; o >>= 1) {
+        const int v = __shfl_xor(mx, o);
+        mx = v > mx ? v : mx;
+    }
+    if (lane == 0) wm[w] = mx;
+    __syncthreads();
+    if (t == 0) {
+        for (int k = 1; k < 16; k++) mx = wm[k] > mx ? wm[k] : mx;
+        offset[ncells] = base;
+        st[0] = mx;
+        st[1] = 0;
+        if (esteps) {
+            esteps[0] = tot[0];
+            esteps[1] = tot[1];
+            esteps[2] = tot[2];
+            esteps[3] = ke;
+        }
+    }
 }
 
 /* The wrapped coordinates l-1, l, l+1 of one axis in ascending order; a
@@ -269,55 +327,87 @@ __device__ __forceinline__ void sorted3(int l, int cdim, int *s) {
     s[2] = c;
 }
 
-/* Arrivals, one thread per destination cell: appended after the stayers in
-   the host's order, by source cell id and then departure order (the source
+/* The new layout, one wave per cell: its stayers, then its arrivals in the
+   host's order, by source cell id and then departure order (the source
    cells' ids ascend with their wrapped coordinates taken in lexicographic
-   order).  Sets st[1] when an arrival is still outside its new cell. */
-__global__ __launch_bounds__(128) void k_arrive(struct step_geom G, const int *__restrict__ old_off,
+   order, lane 9 i + 3 j + k's).  Sets st[1] when an arrival is still outside
+   its new cell.  With pack, also the next pass's FP32 positions, id -> slot
+   and slot -> cell maps, while the atoms are at hand (k_pack's work: 1,048,576
+   atoms, stayers, arrivals, id clearing and packing took 58 us in four
+   launches, this one 36; 32,000 atoms 25 and 6). */
+__global__ __launch_bounds__(256) void k_settle(struct step_geom G, const int *__restrict__ old_cnt,
+                                                const int *__restrict__ old_off, const int *__restrict__ slot,
                                                 const int *__restrict__ ndep, const int *__restrict__ qsrc,
                                                 const int *__restrict__ qdest, const int *__restrict__ new_off,
                                                 const int *__restrict__ stay, const double *__restrict__ x,
                                                 const double *__restrict__ v, const int *__restrict__ id,
                                                 const int *__restrict__ type, double *__restrict__ x2,
                                                 double *__restrict__ v2, int *__restrict__ id2,
-                                                int *__restrict__ type2, int *__restrict__ st) {
+                                                int *__restrict__ type2, int *__restrict__ st, int pack,
+                                                float4 *__restrict__ xf, int *__restrict__ index_of_id,
+                                                int *__restrict__ cell_of, int *__restrict__ queue) {
 #pragma clang fp contract(off)
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    const int c = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (pack && blockIdx.x == 0 && threadIdx.x < MD_NQUEUE) queue[threadIdx.x] = 0;
     if (c >= G.ncells) return;
-    const int loc[3] = {c / (G.cdim[1] * G.cdim[2]), (c / G.cdim[2]) % G.cdim[1], c % G.cdim[2]};
-    int I[3], J[3], K[3];
-    sorted3(loc[0], G.cdim[0], I);
-    sorted3(loc[1], G.cdim[1], J);
-    sorted3(loc[2], G.cdim[2], K);
-    int b = new_off[c] + stay[c], outside = 0;
-#pragma unroll
-    for (int qi = 0; qi < 3; qi++) {
-        if (qi > 0 && I[qi] == I[qi - 1]) continue;
-#pragma unroll
-        for (int qj = 0; qj < 3; qj++) {
-            if (qj > 0 && J[qj] == J[qj - 1]) continue;
-#pragma unroll
-            for (int qk = 0; qk < 3; qk++) {
-                if (qk > 0 && K[qk] == K[qk - 1]) continue;
-                const int s = (I[qi] * G.cdim[1] + J[qj]) * G.cdim[2] + K[qk];
-                const int off = old_off[s], nd = ndep[s];
-                for (int q = off; q < off + nd; q++) {
-                    if (qdest[q] != c) continue;
-                    const int a = off + qsrc[q];
-                    for (int m = 0; m < 3; m++) {
-                        const double xm = x[3 * a + m];
-                        const int d = (xm >= G.h[m]) - (xm < 0.0);
-                        const double xn = xm - d * G.h[m];
-                        x2[3 * b + m] = xn;
-                        v2[3 * b + m] = v[3 * a + m];
-                        outside |= (xn >= G.h[m]) | (xn < 0.0);
-                    }
-                    id2[b] = id[a];
-                    type2[b] = type[a];
-                    b++;
-                }
-            }
+    auto put = [&](int a, int b, const double *xn) {
+        const int i = id[a], t = type[a];
+        for (int m = 0; m < 3; m++) {
+            x2[3 * (size_t)b + m] = xn[m];
+            v2[3 * (size_t)b + m] = v[3 * (size_t)a + m];
         }
+        id2[b] = i;
+        type2[b] = t;
+        if (pack) {
+            xf[b] = make_float4((float)xn[0], (float)xn[1], (float)xn[2], __int_as_float(t));
+            index_of_id[i] = b;
+            cell_of[b] = c;
+        }
+    };
+    const int nb = new_off[c], off = old_off[c], n = old_cnt[c];
+    for (int k = lane; k < n; k += 64) {
+        const int a = off + k, r = slot[a];
+        if (r < 0) continue;
+        const double xa[3] = {x[3 * (size_t)a], x[3 * (size_t)a + 1], x[3 * (size_t)a + 2]};
+        put(a, nb + r, xa);
+    }
+    const int loc[3] = {c / (G.cdim[1] * G.cdim[2]), (c / G.cdim[2]) % G.cdim[1], c % G.cdim[2]};
+    int src = 0, soff = 0, nd = 0, na = 0;
+    if (lane < 27) {
+        const int q[3] = {lane / 9, (lane / 3) % 3, lane % 3};
+        bool repeat = false;
+        for (int m = 0; m < 3; m++) {
+            int w[3];
+            sorted3(loc[m], G.cdim[m], w);
+            const int s = q[m] == 0 ? w[0] : q[m] == 1 ? w[1] : w[2];
+            repeat |= (q[m] == 1 && w[1] == w[0]) || (q[m] == 2 && w[2] == w[1]);
+            src = src * G.cdim[m] + s;
+        }
+        if (!repeat) {
+            soff = old_off[src];
+            nd = ndep[src];
+        }
+        for (int k = soff; k < soff + nd; k++) na += qdest[k] == c;
+    }
+    int upto = na;
+    for (int o = 1; o < 32; o <<= 1) {
+        const int u = __shfl_up(upto, o);
+        if (lane >= o) upto += u;
+    }
+    int b = nb + stay[c] + upto - na;
+    bool outside = false;
+    for (int k = soff; na > 0 && k < soff + nd; k++) {
+        if (qdest[k] != c) continue;
+        const int a = soff + qsrc[k];
+        double xn[3];
+        for (int m = 0; m < 3; m++) {
+            const double xm = x[3 * (size_t)a + m];
+            const int d = (xm >= G.h[m]) - (xm < 0.0);
+            xn[m] = xm - d * G.h[m];
+            outside |= (xn[m] >= G.h[m]) | (xn[m] < 0.0);
+        }
+        put(a, b, xn);
+        b++;
     }
     if (outside) st[1] = 1;
 }
@@ -334,7 +424,8 @@ __global__ __launch_bounds__(64) void k_advance_verlet(int kick, double dt, cons
                                                        const int *__restrict__ count, const int *__restrict__ offset,
                                                        double *__restrict__ x, double *__restrict__ v,
                                                        const int *__restrict__ type, const double *__restrict__ oldx,
-                                                       double *__restrict__ lmax2, double *__restrict__ cell_ke) {
+                                                       double *__restrict__ lmax2, double *__restrict__ cell_ke,
+                                                       float4 *__restrict__ xf) {
 #pragma clang fp contract(off)
     const int c = blockIdx.x, lane = threadIdx.x;
     const int off = offset[c], n = count[c];
@@ -355,6 +446,8 @@ __global__ __launch_bounds__(64) void k_advance_verlet(int kick, double dt, cons
                 v[3 * a + m] = vv[m];
                 x[3 * a + m] = xa[m];
             }
+            /* the next pass's FP32 positions (the layout stays) */
+            if (xf) xf[a] = make_float4((float)xa[0], (float)xa[1], (float)xa[2], __int_as_float(t));
             ke += 0.5 * mass[t] * (vv[0] * vv[0] + vv[1] * vv[1] + vv[2] * vv[2]);
         } else {
             const double m = mass[type[a]], v0 = v[3 * a], v1 = v[3 * a + 1], v2 = v[3 * a + 2];
@@ -618,22 +711,28 @@ __global__ __launch_bounds__(128) void k_rigid(struct rigid_dev R, int shake, in
 
 struct step_bufs {
     double *v, *x2, *v2, *mass, *imass, *cell_ke, *bke, *esteps;
-    double *oldx, *lmax2, *bmx, *vmax; /* pseudo-Verlet */
+    double *oldx, *lmax2, *bmx; /* pseudo-Verlet */
+    /* pinned host memory that the kernels write to: largest cell count and
+       outside flag of a migration, largest squared displacement */
+    int *st;
+    double *vmax;
     /* rigid groups: device copies, slot of each id, P-SHAKE forces by id */
     int *rg_np, *rg_nc, *rg_parts, *rg_ij, *sid;
     double *rg_d2, *fcorr;
     float *rg_a;
     int nrig;
-    int *id2, *type2, *slot, *qsrc, *qdest, *stay, *ndep, *narr, *bsum, *bmax, *st, *count2, *offset2;
+    int *id2, *type2, *slot, *qsrc, *qdest, *stay, *ndep, *narr, *bsum, *bmax, *count2, *offset2;
     int nblocks;
 };
 
 static void step_free(struct step_bufs *b) {
     double *d[] = {b->v, b->x2, b->v2, b->mass, b->imass, b->cell_ke, b->bke, b->esteps,
-                   b->oldx, b->lmax2, b->bmx, b->vmax, b->rg_d2, b->fcorr};
+                   b->oldx, b->lmax2, b->bmx, b->rg_d2, b->fcorr};
     int *i[] = {b->id2, b->type2, b->slot, b->qsrc, b->qdest, b->stay, b->ndep, b->narr, b->bsum,
-                b->bmax, b->st, b->count2, b->offset2, b->rg_np, b->rg_nc, b->rg_parts, b->rg_ij, b->sid};
+                b->bmax, b->count2, b->offset2, b->rg_np, b->rg_nc, b->rg_parts, b->rg_ij, b->sid};
     (void)hipFree(b->rg_a);
+    (void)hipHostFree(b->st);
+    (void)hipHostFree(b->vmax);
     for (size_t k = 0; k < sizeof(d) / sizeof(d[0]); k++) (void)hipFree(d[k]);
     for (size_t k = 0; k < sizeof(i) / sizeof(i[0]); k++) (void)hipFree(i[k]);
     memset(b, 0, sizeof(*b));
@@ -656,11 +755,12 @@ static int step_alloc(struct step_bufs *b, size_t N, int ncells, int ntypes, int
         hipMalloc(&b->qdest, sizeof(int) * N) != hipSuccess || hipMalloc(&b->stay, sizeof(int) * C) != hipSuccess ||
         hipMalloc(&b->ndep, sizeof(int) * C) != hipSuccess || hipMalloc(&b->narr, sizeof(int) * C) != hipSuccess ||
         hipMalloc(&b->bsum, sizeof(int) * B) != hipSuccess || hipMalloc(&b->bmax, sizeof(int) * B) != hipSuccess ||
-        hipMalloc(&b->st, sizeof(int) * 2) != hipSuccess || hipMalloc(&b->count2, sizeof(int) * C) != hipSuccess ||
+        hipHostMalloc((void **)&b->st, sizeof(int) * 2, hipHostMallocDefault) != hipSuccess ||
+        hipMalloc(&b->count2, sizeof(int) * C) != hipSuccess ||
         hipMalloc(&b->offset2, sizeof(int) * (C + 1)) != hipSuccess ||
         hipMalloc(&b->oldx, sizeof(double) * 3 * N) != hipSuccess ||
         hipMalloc(&b->lmax2, sizeof(double) * C) != hipSuccess || hipMalloc(&b->bmx, sizeof(double) * B) != hipSuccess ||
-        hipMalloc(&b->vmax, sizeof(double)) != hipSuccess ||
+        hipHostMalloc((void **)&b->vmax, sizeof(double), hipHostMallocDefault) != hipSuccess ||
         hipMemset(b->narr, 0, sizeof(int) * C) != hipSuccess) {
         step_free(b);
         return -1;
@@ -729,26 +829,31 @@ void gpu_steps_free(struct gpu_state *g) {
 
 /* Shuffle (es == NULL: no kick) or advance (kick-drift, then migration, the
    step's energies into es[0..3]): departures, the new layout, stayers and
-   arrivals copied into it, then the layouts swapped.  Asynchronous; the
-   largest new cell count and the outside flag land in b->st. */
+   arrivals copied into it (pack: and into the next pass's arrays), then the
+   layouts swapped.  Asynchronous; the largest new cell count and the outside
+   flag land in b->st once g->ev[4] has passed. */
 static int step_migrate(struct gpu_state *g, struct step_bufs *b, const struct step_geom &G, double dt,
-                        double *es) {
-    const int n = g->nparts, nc = g->ncells, kick = es != NULL;
-    const int nbp = n > 0 ? (n + 255) / 256 : 1;
+                        double *es, int pack) {
+    const int nc = g->ncells, kick = es != NULL;
+    const double *cell_ke = kick ? b->cell_ke : NULL;
     hipLaunchKernelGGL(k_migrate, dim3(nc), dim3(64), 0, g->stream, G, kick, dt, b->mass, b->imass, g->d_fhi,
-                       g->d_flo, g->d_count, g->d_offset, g->d_x, b->v, g->d_type, g->d_cell_of, b->slot, b->qsrc,
-                       b->qdest, b->stay, b->ndep, b->narr, b->cell_ke);
-    hipLaunchKernelGGL(k_scan_a, dim3(b->nblocks), dim3(256), 0, g->stream, nc, b->stay, b->narr,
-                       kick ? b->cell_ke : (const double *)NULL, b->bsum, b->bmax, b->bke);
-    hipLaunchKernelGGL(k_scan_b, dim3(1), dim3(64), 0, g->stream, b->nblocks, nc, b->bsum, b->bmax, b->bke,
-                       b->offset2, b->st, g->d_tot, es);
-    hipLaunchKernelGGL(k_scan_c, dim3(b->nblocks), dim3(256), 0, g->stream, nc, b->stay, b->narr, b->bsum,
-                       b->count2, b->offset2, g->d_cnt_off);
-    hipLaunchKernelGGL(k_stayers, dim3(nbp), dim3(256), 0, g->stream, n, g->d_cell_of, b->slot, b->offset2, g->d_x,
-                       b->v, g->d_id, g->d_type, b->x2, b->v2, b->id2, b->type2);
-    hipLaunchKernelGGL(k_arrive, dim3((nc + 127) / 128), dim3(128), 0, g->stream, G, g->d_offset, b->ndep, b->qsrc,
-                       b->qdest, b->offset2, b->stay, g->d_x, b->v, g->d_id, g->d_type, b->x2, b->v2, b->id2,
-                       b->type2, b->st);
+                       g->d_flo, g->d_count, g->d_offset, g->d_x, b->v, g->d_type, b->slot, b->qsrc, b->qdest,
+                       b->stay, b->ndep, b->narr, b->cell_ke);
+    if (nc <= MD_SCAN_ONE)
+        hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(1024), 0, g->stream, nc, b->stay, b->narr, cell_ke, b->count2,
+                           b->offset2, g->d_cnt_off, b->st, g->d_tot, es);
+    else {
+        hipLaunchKernelGGL(k_scan_a, dim3(b->nblocks), dim3(256), 0, g->stream, nc, b->stay, b->narr, cell_ke, b->bsum,
+                           b->bmax, b->bke);
+        hipLaunchKernelGGL(k_scan_b, dim3(1), dim3(64), 0, g->stream, b->nblocks, nc, b->bsum, b->bmax, b->bke,
+                           b->offset2, b->st, g->d_tot, es);
+        hipLaunchKernelGGL(k_scan_c, dim3(b->nblocks), dim3(256), 0, g->stream, nc, b->stay, b->narr, b->bsum,
+                           b->count2, b->offset2, g->d_cnt_off);
+    }
+    hipLaunchKernelGGL(k_settle, dim3((nc + 3) / 4), dim3(256), 0, g->stream, G, g->d_count, g->d_offset, b->slot,
+                       b->ndep, b->qsrc, b->qdest, b->offset2, b->stay, g->d_x, b->v, g->d_id, g->d_type, b->x2, b->v2,
+                       b->id2, b->type2, b->st, pack, g->d_xf, g->d_index_of_id, g->d_cell_of, g->d_queue);
+    HIPCHECK(hipEventRecord(g->ev[4], g->stream));
     HIPCHECK(hipGetLastError());
     double *t;
     int *u;
@@ -761,13 +866,11 @@ static int step_migrate(struct gpu_state *g, struct step_bufs *b, const struct s
     return engine_err_ok;
 }
 
-/* Wait for the last migration; its largest cell count and whether an
-   arrival is still outside its cell. */
+/* Wait for the last migration (and the constraints after it); its largest
+   cell count and whether an arrival is still outside its cell. */
 static int step_status(struct gpu_state *g, struct step_bufs *b, int *maxc, int *outside) {
-    int st[2];
-    if (hipMemcpyAsync(st, b->st, sizeof(st), hipMemcpyDeviceToHost, g->stream) != hipSuccess ||
-        hipStreamSynchronize(g->stream) != hipSuccess)
-        return gerror_(engine_err_gpu, "migration failed");
+    if (hipEventSynchronize(g->ev[4]) != hipSuccess) return gerror_(engine_err_gpu, "migration failed");
+    const volatile int *st = b->st;
     *maxc = st[0];
     *outside = st[1];
     if (st[0] > g->maxcell) return gerror_(engine_err_maxparts, "more particles in a cell than the packed record holds");
@@ -975,22 +1078,30 @@ static int rigid_step(struct engine *e, struct gpu_state *g, struct step_bufs *b
                        (e->flags & engine_flag_shake) != 0, (e->time + 1) < engine_pshake_steps, e->dt, e->tol_rigid,
                        G, b->mass, b->sid, g->d_cell_of, g->d_type, g->d_x, b->v, b->fcorr, b->st);
     hipLaunchKernelGGL(k_advance_verlet, dim3(nc), dim3(64), 0, g->stream, 0, 0.0, b->mass, b->imass, g->d_fhi,
-                       g->d_flo, g->d_count, g->d_offset, g->d_x, b->v, g->d_type, oldx, b->lmax2, b->cell_ke);
+                       g->d_flo, g->d_count, g->d_offset, g->d_x, b->v, g->d_type, oldx, b->lmax2, b->cell_ke,
+                       (float4 *)NULL);
     hipLaunchKernelGGL(k_verlet_red_a, dim3(b->nblocks), dim3(256), 0, g->stream, nc, b->cell_ke, b->lmax2, b->bke,
                        b->bmx);
     hipLaunchKernelGGL(k_verlet_red_b, dim3(1), dim3(64), 0, g->stream, b->nblocks, b->bke, b->bmx, g->d_tot, es,
                        b->vmax);
-    if (hipGetLastError() != hipSuccess) return gerror_(engine_err_gpu, "constraints failed");
+    if (hipGetLastError() != hipSuccess || hipEventRecord(g->ev[4], g->stream) != hipSuccess)
+        return gerror_(engine_err_gpu, "constraints failed");
     return engine_err_ok;
 }
 
-/* Largest squared displacement of the last k_advance_verlet. */
+/* Largest squared displacement of the last k_advance_verlet (before ev[4]). */
 static int verlet_status(struct gpu_state *g, struct step_bufs *b, double *vmax) {
-    if (hipMemcpyAsync(vmax, b->vmax, sizeof(double), hipMemcpyDeviceToHost, g->stream) != hipSuccess ||
-        hipStreamSynchronize(g->stream) != hipSuccess)
-        return gerror_(engine_err_gpu, "advance failed");
+    if (hipEventSynchronize(g->ev[4]) != hipSuccess) return gerror_(engine_err_gpu, "advance failed");
+    *vmax = *(const volatile double *)b->vmax;
     return engine_err_ok;
 }
+
+/* Whether a step's pass may be launched before the status of the migration or
+   advance before it is known (the device would else wait 25 to 30 us a step
+   for the host): k_pair's pass, which changes nothing but its own results and
+   stays inside its arrays whatever the cells hold.  The other pair kernels'
+   LDS is sized by the largest cell. */
+static int steps_ahead(const struct gpu_state *g, int mlp) { return !mlp && !g->half; }
 
 /* The steps with pseudo-Verlet sort reuse: engine_verlet_update
    (engine.c:193-315) at the start of each step, the pass sorting only on a
@@ -1030,24 +1141,30 @@ static int steps_verlet(struct engine *e, struct gpu_state *g, struct step_bufs 
     if (!rebuild) {
         /* displacements of the uploaded positions */
         hipLaunchKernelGGL(k_advance_verlet, dim3(nc), dim3(64), 0, g->stream, 0, 0.0, b->mass, b->imass, g->d_fhi,
-                           g->d_flo, g->d_count, g->d_offset, g->d_x, b->v, g->d_type, b->oldx, b->lmax2, b->cell_ke);
+                           g->d_flo, g->d_count, g->d_offset, g->d_x, b->v, g->d_type, b->oldx, b->lmax2, b->cell_ke,
+                           (float4 *)NULL);
         hipLaunchKernelGGL(k_verlet_red_a, dim3(b->nblocks), dim3(256), 0, g->stream, nc, b->cell_ke, b->lmax2, b->bke,
                            b->bmx);
         hipLaunchKernelGGL(k_verlet_red_b, dim3(1), dim3(64), 0, g->stream, b->nblocks, b->bke, b->bmx, g->d_tot,
                            (double *)NULL, b->vmax);
+        HIPCHECK(hipEventRecord(g->ev[4], g->stream));
         if ((rc = verlet_status(g, b, &vmax)) < 0) return rc;
     }
+    /* whether the pass's FP32 positions and maps are those of the current
+       particles; whether this step's pass is already under way */
+    int packed = 0, under = 0;
     for (int step = 0; step < nsteps; step++) {
         if (!rebuild) {
             /* engine_verlet_update without a pending rebuild */
-            hipLaunchKernelGGL(k_cell_maxdx, dim3(nbc), dim3(256), 0, g->stream, nc, b->lmax2, g->d_cell_maxdx);
+            if (!under)
+                hipLaunchKernelGGL(k_cell_maxdx, dim3(nbc), dim3(256), 0, g->stream, nc, b->lmax2, g->d_cell_maxdx);
             const double maxdx = sqrt(vmax);
             rebuild = (2.0 * maxdx > skin) || (maxdx > s->cutoff * engine_maxdxratio);
             if (!rebuild) *smaxdx = maxdx;
         }
         if (rebuild) {
             /* engine_shuffle, then the rebuild positions */
-            if ((rc = step_migrate(g, b, G, 0.0, NULL)) < 0 || (rc = step_status(g, b, &maxc, &outside)) < 0) break;
+            if ((rc = step_migrate(g, b, G, 0.0, NULL, 1)) < 0 || (rc = step_status(g, b, &maxc, &outside)) < 0) break;
             if (hipMemcpyAsync(b->oldx, g->d_x, sizeof(double) * 3 * g->nparts, hipMemcpyDeviceToDevice, g->stream) !=
                 hipSuccess) {
                 rc = gerror_(engine_err_gpu, "rebuild failed");
@@ -1056,20 +1173,31 @@ static int steps_verlet(struct engine *e, struct gpu_state *g, struct step_bufs 
             *smaxdx = 0.0;
             g->maxcount = maxc;
             g->P.maxn = maxc > 0 ? maxc : 1;
+            packed = 1;
+            under = 0; /* a pass under way is of the layout before */
         }
-        if ((rc = gpu_launch(g, 0, mlp, rebuild)) < 0) break;
+        if (!under && (rc = gpu_launch(g, 0, mlp, rebuild, packed)) < 0) break;
         rebuild = 0;
         hipLaunchKernelGGL(k_advance_verlet, dim3(nc), dim3(64), 0, g->stream, 1, e->dt, b->mass, b->imass, g->d_fhi,
-                           g->d_flo, g->d_count, g->d_offset, g->d_x, b->v, g->d_type, b->oldx, b->lmax2, b->cell_ke);
+                           g->d_flo, g->d_count, g->d_offset, g->d_x, b->v, g->d_type, b->oldx, b->lmax2, b->cell_ke,
+                           g->d_xf);
         hipLaunchKernelGGL(k_verlet_red_a, dim3(b->nblocks), dim3(256), 0, g->stream, nc, b->cell_ke, b->lmax2, b->bke,
                            b->bmx);
         hipLaunchKernelGGL(k_verlet_red_b, dim3(1), dim3(64), 0, g->stream, b->nblocks, b->bke, b->bmx, g->d_tot,
                            b->esteps + 4 * step, b->vmax);
-        if (hipGetLastError() != hipSuccess) {
+        if (hipGetLastError() != hipSuccess || hipEventRecord(g->ev[4], g->stream) != hipSuccess) {
             rc = gerror_(engine_err_gpu, "advance failed");
             break;
         }
+        packed = b->nrig == 0; /* the constraints move particles once more */
         if (b->nrig > 0 && (rc = rigid_step(e, g, b, G, b->oldx, b->esteps + 4 * step)) < 0) break;
+        /* the next step's pass before its status is known: right unless that
+           step rebuilds, which does it over */
+        under = packed && step + 1 < nsteps && steps_ahead(g, mlp);
+        if (under) {
+            hipLaunchKernelGGL(k_cell_maxdx, dim3(nbc), dim3(256), 0, g->stream, nc, b->lmax2, g->d_cell_maxdx);
+            if ((rc = gpu_launch(g, 0, mlp, 0, 1)) < 0) break;
+        }
         if ((rc = verlet_status(g, b, &vmax)) < 0) break;
         e->time += 1;
     }
@@ -1122,24 +1250,47 @@ extern "C" int engine_gpu_steps(struct engine *e, int nsteps, double *epot, doub
     const int verlet = (e->flags & engine_flag_verlet) != 0;
     double smaxdx = s->maxdx;
     if (rc == engine_err_ok) rc = rigid_upload(e, g, &b);
+    if (rc == engine_err_ok && gpu_clear_ids(g) < 0) rc = engine_err_gpu;
     if (verlet && rc == engine_err_ok)
         rc = steps_verlet(e, g, &b, G, nsteps, &smaxdx);
     /* engine_step: shuffle, pass, advance.  After an advance that left every
        particle inside its cell, the next shuffle moves nothing and is skipped. */
+    const int mlp = (e->flags & engine_flag_mlp) != 0, pack = b.nrig == 0;
+    int under = 0; /* this step's pass is under way, with cells of up to g->maxcount sorted */
     outside = 1;
     for (int step = 0; step < nsteps && rc == engine_err_ok && !verlet; step++) {
         if (outside) {
-            if ((rc = step_migrate(g, &b, G, 0.0, NULL)) < 0 || (rc = step_status(g, &b, &maxc, &outside)) < 0)
+            if ((rc = step_migrate(g, &b, G, 0.0, NULL, pack)) < 0 || (rc = step_status(g, &b, &maxc, &outside)) < 0)
                 break;
+            under = 0;
         }
+        if (!under || maxc > g->maxcount) {
+            g->maxcount = maxc;
+            g->P.maxn = maxc > 0 ? maxc : 1;
+            if ((rc = gpu_launch(g, 0, mlp, 1, pack)) < 0) break;
+        }
+        /* the last pass's id -> slot map goes with its forces: keep it */
+        if ((rc = step_migrate(g, &b, G, e->dt, b.esteps + 4 * step, pack && step + 1 < nsteps)) < 0 ||
+            (b.nrig > 0 && (rc = rigid_step(e, g, &b, G, NULL, b.esteps + 4 * step)) < 0))
+            break;
+        /* the next step's pass before the migration's status is known: right
+           unless a particle is still outside its cell or a cell has grown by
+           more than the margin, which do it over */
+        under = pack && step + 1 < nsteps && steps_ahead(g, mlp);
+        if (under) {
+            int lim = maxc + 4 + maxc / 8;
+            /* not past a limit of the sort's variants, which would only slow it */
+            if (maxc <= MD_SORT_ONEWAVE_MAX && lim > MD_SORT_ONEWAVE_MAX) lim = MD_SORT_ONEWAVE_MAX;
+            if (maxc <= MD_SORT_LDS_MAX && lim > MD_SORT_LDS_MAX) lim = MD_SORT_LDS_MAX;
+            g->maxcount = g->P.maxn = lim;
+            if ((rc = gpu_launch(g, 0, mlp, 1, 1)) < 0) break;
+        }
+        if ((rc = step_status(g, &b, &maxc, &outside)) < 0) break;
+        e->time += 1;
+    }
+    if (!verlet) {
         g->maxcount = maxc;
         g->P.maxn = maxc > 0 ? maxc : 1;
-        if ((rc = gpu_launch(g, 0, (e->flags & engine_flag_mlp) != 0, 1)) < 0) break;
-        if ((rc = step_migrate(g, &b, G, e->dt, b.esteps + 4 * step)) < 0 ||
-            (b.nrig > 0 && (rc = rigid_step(e, g, &b, G, NULL, b.esteps + 4 * step)) < 0) ||
-            (rc = step_status(g, &b, &maxc, &outside)) < 0)
-            break;
-        e->time += 1;
     }
     if (rc == engine_err_ok &&
         (hipMemcpyAsync(&flag, g->d_queue + MD_NQUEUE, sizeof(int), hipMemcpyDeviceToHost, g->stream) != hipSuccess ||
