@@ -12,11 +12,10 @@
  *                  dG1 = W2^T dT2, dW2 = dZ2 H1^T + dT2 G1^T) run on
  *                  v_mfma_f32_16x16x32_bf16 with bf16 operands and fp32
  *                  accumulation; the rest is fp32 VALU.
- *   k_mlp_wsum     fixed-order sum of the per-wave partial rows of the
- *                  shared weights (W2, W1, b2);
- *   k_mlp_tsum     fixed-order sum of the per-tile rows of the per-pair
- *                  parameters (heads W3, b3, the bias gradient of b1e) and
- *                  of the loss, tiles in batch order;
+ *   k_mlp_sums     fixed-order sums: of the per-block partial rows of the
+ *                  shared weights (W2, W1, b2), of the per-tile rows of the
+ *                  per-pair parameters (heads W3, b3, the bias gradient of
+ *                  b1e) and of the loss, tiles in batch order;
  *   k_mlp_chain    gradient of b1, E1 and the embeddings from the gradient
  *                  of the per-pair bias b1e = b1 + E1 emb[p];
  *   k_mlp_adam     Adam on the fp32 master parameters;
@@ -127,8 +126,16 @@ __device__ __forceinline__ float mlp_sum16(float v) {
     return v;
 }
 
-/* One wave per block; each block walks tiles of 16 samples s = 16 t + n,
-   n = 0..15, which all share species pair sp[16 t].  Loss per sample:
+/* A block of MLP_GW waves takes the tiles ti = b, b + G, b + 2 G, ... (G
+   blocks), MLP_GW at a time, one per wave: the forward pass and the backward
+   pass down to the tile's own sums.  What adds up over tiles is then added in
+   tile order, each wave taking a quarter of the sums (16 rows of W2, 4 of the
+   lane's 16 units of W1 and b2) through LDS, so the sums are those of one wave
+   walking the tiles alone.  A tile is one long chain of SiLUs, products and
+   16-lane sums (12 us) and a batch gives each CU a few tiles: one wave per CU
+   took 49 us for 1024 tiles, 4 waves 19.
+   Tile: 16 samples s = 16 t + n, n = 0..15, which all share species pair
+   sp[16 t].  Loss per sample:
    wE (y - a)^2 + wF (yd - ad)^2 / (ad^2 + 1/c^2), a = asinh(E/sE),
    ad = F/sqrt(sE^2 + E^2) its r-derivative for the target's dE/dr = F,
    c = (r_hi - r_lo)/2: the derivative's error relative where |ad| is large
@@ -141,26 +148,34 @@ __device__ __forceinline__ float mlp_sum16(float v) {
      dW1 = dz1 x^T + dt1 (dx/dr)^T,  db1e = dz1,
      dW2 = dz2 h1^T + dt2 g1^T: one MFMA K of 32 per tile, the 16 value
      columns and the 16 derivative columns (through LDS).
-   Sums over the shared weights go to this wave's partial row, those of the
+   Sums over the shared weights go to the block's partial row, those of the
    tile's pair to the tile's row of tpart (index ti of tiles[]).  A pair id
    outside [0, np) is read as pair 0 and sets *err. */
-__global__ __launch_bounds__(64) void k_mlp_grad(struct mlp_net N, const float *__restrict__ sr,
+#define MLP_GW 4
+__global__ __launch_bounds__(64 * MLP_GW) void k_mlp_grad(struct mlp_net N, const float *__restrict__ sr,
                                                  const int *__restrict__ sp, const float *__restrict__ tE,
                                                  const float *__restrict__ tF, const int *__restrict__ tiles,
                                                  int ntiles, float wE, float wF, float inv_n, int np,
                                                  float *__restrict__ tpart, float *__restrict__ partial,
                                                  float *__restrict__ err) {
-    __shared__ __attribute__((aligned(16))) __bf16 h1t[MLP_H][32]; /* [in unit][h1 of 16 samples, g1 of 16]   */
-    __shared__ __attribute__((aligned(16))) __bf16 dzt[MLP_H][32]; /* [out unit][dz2 of 16 samples, dt2 of 16] */
-    const int lane = threadIdx.x, n = lane & 15, g = lane >> 4;
-    mlp_f4 dw2[16];
-    float dw1a[16], dw1b[16], db2[16];
+    /* per wave's tile: [in unit][h1 of 16 samples, g1 of 16], [out unit][dz2
+       of 16 samples, dt2 of 16]; dz1, dt1, dz2 by unit and lane; inputs */
+    __shared__ __attribute__((aligned(16))) __bf16 h1s[MLP_GW][MLP_H][32], dzs[MLP_GW][MLP_H][32];
+    __shared__ float dz1s[MLP_GW][16][64], dt1s[MLP_GW][16][64], dz2s[MLP_GW][16][64];
+    __shared__ float4 ins[MLP_GW][16];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = lane & 15, g = lane >> 4;
+    mlp_f4 dw2[4];
+    float dw1a[4], dw1b[4], db2[4];
 #pragma unroll
-    for (int q = 0; q < 16; q++) {
+    for (int q = 0; q < 4; q++) {
         dw2[q] = (mlp_f4){0.f, 0.f, 0.f, 0.f};
         dw1a[q] = dw1b[q] = db2[q] = 0.f;
     }
-    for (int ti = blockIdx.x; ti < ntiles; ti += gridDim.x) {
+    for (int t0 = blockIdx.x; t0 < ntiles; t0 += MLP_GW * gridDim.x) {
+        const int ti = t0 + wave * (int)gridDim.x;
+        const int nt = min(MLP_GW, (ntiles - t0 + (int)gridDim.x - 1) / (int)gridDim.x); /* tiles of this round */
+        if (ti < ntiles) {
+        __bf16 (*const h1t)[32] = h1s[wave], (*const dzt)[32] = dzs[wave];
         const int tile = tiles[ti];
         const int s = 16 * tile + n;
         int p = sp[16 * tile];
@@ -198,7 +213,7 @@ __global__ __launch_bounds__(64) void k_mlp_grad(struct mlp_net N, const float *
             mlp_silu3(z2[j], h, d, dd);
             dz2[j] = w * (dy * d + dyd * t2[j] * dd);
             dt2[j] = w * dyd * d;
-            db2[j] += dz2[j];
+            dz2s[wave][j][lane] = dz2[j];
             const float gw = mlp_sum16(dy * h + dyd * d * t2[j]);
             if (n == 0) trow[u] = gw;
         }
@@ -218,6 +233,7 @@ __global__ __launch_bounds__(64) void k_mlp_grad(struct mlp_net N, const float *
             }
         float rn, irn, drn, dirn;
         mlp_inputs(sc, r, rn, irn, drn, dirn);
+        if (g == 0) ins[wave][n] = make_float4(rn, irn, drn, dirn);
 #pragma unroll
         for (int mb = 0; mb < 4; mb++) {
             const mlp_bf16x8 a0 = N.w2b[(mb * 2 + 0) * 64 + lane], a1 = N.w2b[(mb * 2 + 1) * 64 + lane];
@@ -233,8 +249,8 @@ __global__ __launch_bounds__(64) void k_mlp_grad(struct mlp_net N, const float *
                 mlp_silu3(z1[j], h, d, dd);
                 const float dz1 = acc[i] * d + act[i] * t1[j] * dd;
                 const float dt1 = act[i] * d;
-                dw1a[j] += dz1 * rn + dt1 * drn;
-                dw1b[j] += dz1 * irn + dt1 * dirn;
+                dz1s[wave][j][lane] = dz1;
+                dt1s[wave][j][lane] = dt1;
                 const float gsum = mlp_sum16(dz1);
                 if (n == 0) trow[MLP_TR_B1E + mlp_unit(j, lane)] = gsum;
             }
@@ -249,33 +265,41 @@ __global__ __launch_bounds__(64) void k_mlp_grad(struct mlp_net N, const float *
             dzt[u][n] = dzb[j >> 3][j & 7];
             dzt[u][16 + n] = dtb[j >> 3][j & 7];
         }
+        }
         __syncthreads();
-        /* dW2[m][k] += sum over the 32 columns of dZ2|dT2[m] H1|G1[k]. */
-#pragma unroll
-        for (int mb = 0; mb < 4; mb++) {
-            const mlp_bf16x8 a = *(const mlp_bf16x8 *)&dzt[16 * mb + n][8 * g];
+        for (int k = 0; k < nt; k++) {
+            /* dW2[m][k] += sum over the 32 columns of dZ2|dT2[m] H1|G1[k], rows
+               of block m = wave. */
+            const mlp_bf16x8 a = *(const mlp_bf16x8 *)&dzs[k][16 * wave + n][8 * g];
 #pragma unroll
             for (int kb = 0; kb < 4; kb++) {
-                const mlp_bf16x8 b = *(const mlp_bf16x8 *)&h1t[16 * kb + n][8 * g];
-                dw2[mb * 4 + kb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, dw2[mb * 4 + kb], 0, 0, 0);
+                const mlp_bf16x8 b = *(const mlp_bf16x8 *)&h1s[k][16 * kb + n][8 * g];
+                dw2[kb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, dw2[kb], 0, 0, 0);
+            }
+            const float4 in = ins[k][n];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int j = 4 * wave + i;
+                const float dz1 = dz1s[k][j][lane], dt1 = dt1s[k][j][lane];
+                dw1a[i] += fmaf(dt1, in.z, dz1 * in.x);
+                dw1b[i] += fmaf(dt1, in.w, dz1 * in.y);
+                db2[i] += dz2s[k][j][lane];
             }
         }
         __syncthreads();
     }
 
-    /* This wave's sums of the shared weights go to its own partial row
-       (summed over waves in a fixed order by k_mlp_wsum): W2, then W1, b2. */
+    /* The block's sums of the shared weights go to its own partial row
+       (summed over blocks in a fixed order by k_mlp_sums): W2, then W1, b2. */
     float *row = partial + (size_t)blockIdx.x * MLP_WPART;
 #pragma unroll
-    for (int mb = 0; mb < 4; mb++)
+    for (int kb = 0; kb < 4; kb++)
 #pragma unroll
-        for (int kb = 0; kb < 4; kb++)
+        for (int i = 0; i < 4; i++) row[(16 * wave + 4 * g + i) * MLP_H + 16 * kb + n] = dw2[kb][i];
 #pragma unroll
-            for (int i = 0; i < 4; i++) row[(16 * mb + 4 * g + i) * MLP_H + 16 * kb + n] = dw2[mb * 4 + kb][i];
-#pragma unroll
-    for (int j = 0; j < 16; j++) {
-        const int u = mlp_unit(j, lane);
-        const float a = mlp_sum16(dw1a[j]), b = mlp_sum16(dw1b[j]), c = mlp_sum16(db2[j]);
+    for (int i = 0; i < 4; i++) {
+        const int u = mlp_unit(4 * wave + i, lane);
+        const float a = mlp_sum16(dw1a[i]), b = mlp_sum16(dw1b[i]), c = mlp_sum16(db2[i]);
         if (n == 0) {
             row[MLP_H * MLP_H + 2 * u] = a;
             row[MLP_H * MLP_H + 2 * u + 1] = b;
@@ -284,63 +308,85 @@ __global__ __launch_bounds__(64) void k_mlp_grad(struct mlp_net N, const float *
     }
 }
 
-/* Sum the per-wave partial rows of k_mlp_grad into the gradient.  Block b
-   takes columns [64 b, 64 b + 64); its wave s sums rows s, s + MLP_WSUM_SPLIT,
-   ... in order, and the MLP_WSUM_SPLIT sums are then added in wave order, so
-   every run gives the same bits.  (One thread per column summing all rows
-   left 17 blocks each waiting on ~500 dependent loads: 113 us per step.) */
+/* Sum the partial rows of k_mlp_grad into the gradient; with add into what is
+   there (a later chunk of tiles), else in its place.
+   Blocks b < MLP_WBLOCKS, the shared weights: columns [64 b, 64 b + 64); wave
+   s sums rows s, s + MLP_WSUM_SPLIT, ... in order, and the MLP_WSUM_SPLIT sums
+   are then added in wave order, so every run gives the same bits.
+   Blocks MLP_WBLOCKS + p, p < np: the rows of the tiles of pair p, in tile
+   order, into the gradients of its heads and b1e.  The block lists its tiles
+   first (ballots, in order): walking all tiles and testing each took 52 us for
+   1024 tiles of 210 pairs, one dependent LDS read after the other, and the
+   shared weights 6 in another launch; all of this takes 5.3.
+   Block MLP_WBLOCKS + np: the tiles' losses (thread k < 256 takes tiles k,
+   k + 256, ... in order, then a fixed tree).  A pair id outside [0, np) marks
+   no tile; with *err set the loss becomes NaN. */
 #define MLP_WSUM_SPLIT 16
-__global__ __launch_bounds__(64 * MLP_WSUM_SPLIT) void k_mlp_wsum(const float *__restrict__ partial, int nwaves,
-                                                                  float *__restrict__ grad) {
+#define MLP_WBLOCKS ((MLP_WPART + 63) / 64)
+__global__ __launch_bounds__(64 * MLP_WSUM_SPLIT) void k_mlp_sums(const float *__restrict__ partial, int nrows,
+                                                                  const float *__restrict__ tpart,
+                                                                  const int *__restrict__ tiles, int ntiles,
+                                                                  const int *__restrict__ sp, int np, int add,
+                                                                  float *__restrict__ grad, float *__restrict__ gb1e,
+                                                                  float *__restrict__ loss,
+                                                                  const float *__restrict__ err) {
     __shared__ float part[MLP_WSUM_SPLIT][64];
-    const int col = threadIdx.x & 63, s = threadIdx.x >> 6;
-    const int t = blockIdx.x * 64 + col;
-    float acc = 0.f;
-    if (t < MLP_WPART)
-        for (int w = s; w < nwaves; w += MLP_WSUM_SPLIT) acc += partial[(size_t)w * MLP_WPART + t];
-    part[s][col] = acc;
-    __syncthreads();
-    if (s != 0 || t >= MLP_WPART) return;
-    acc = 0.f;
-    for (int k = 0; k < MLP_WSUM_SPLIT; k++) acc += part[k][col];
-    if (t < MLP_H * MLP_H)
-        grad[MLP_OFF_W2 + t] += acc;
-    else if (t < MLP_H * MLP_H + 2 * MLP_H)
-        grad[MLP_OFF_W1 + t - MLP_H * MLP_H] += acc;
-    else
-        grad[MLP_OFF_B2 + t - MLP_H * MLP_H - 2 * MLP_H] += acc;
-}
-
-/* Add the per-tile rows of k_mlp_grad: block p < np sums the rows of the
-   tiles of pair p, in tile order, into the gradients of its heads and
-   b1e; block np sums the tiles' losses (thread k takes tiles k, k + 256,
-   ... in order, then a fixed tree).  A pair id outside [0, np) marks no
-   tile; with *err set the loss becomes NaN. */
-__global__ __launch_bounds__(256) void k_mlp_tsum(const float *__restrict__ tpart, const int *__restrict__ tiles,
-                                                  int ntiles, const int *__restrict__ sp, int np,
-                                                  float *__restrict__ grad, float *__restrict__ gb1e,
-                                                  float *__restrict__ loss, const float *__restrict__ err) {
-    __shared__ unsigned char mine[MLP_TCHUNK];
-    __shared__ float red[256];
-    const int p = blockIdx.x, c = threadIdx.x;
-    if (p < np) {
-        for (int t = c; t < ntiles; t += 256) mine[t] = sp[16 * tiles[t]] == p;
+    __shared__ unsigned short list[MLP_TCHUNK];
+    __shared__ int cnt[MLP_WSUM_SPLIT];
+    const int c = threadIdx.x, lane = c & 63, s = c >> 6, p = (int)blockIdx.x - MLP_WBLOCKS;
+    auto put = [add](float *d, float v) { *d = (add ? *d : 0.0f) + v; };
+    if (p < 0) {
+        const int t = blockIdx.x * 64 + lane;
+        float acc = 0.f;
+        if (t < MLP_WPART) {
+#pragma unroll 4
+            for (int w = s; w < nrows; w += MLP_WSUM_SPLIT) acc += partial[(size_t)w * MLP_WPART + t];
+        }
+        part[s][lane] = acc;
         __syncthreads();
+        if (s != 0 || t >= MLP_WPART) return;
+        acc = 0.f;
+        for (int k = 0; k < MLP_WSUM_SPLIT; k++) acc += part[k][lane];
+        if (t < MLP_H * MLP_H)
+            put(&grad[MLP_OFF_W2 + t], acc);
+        else if (t < MLP_H * MLP_H + 2 * MLP_H)
+            put(&grad[MLP_OFF_W1 + t - MLP_H * MLP_H], acc);
+        else
+            put(&grad[MLP_OFF_B2 + t - MLP_H * MLP_H - 2 * MLP_H], acc);
+    } else if (p < np) {
+        int nl = 0;
+        for (int t0 = 0; t0 < ntiles; t0 += 64 * MLP_WSUM_SPLIT) {
+            const int t = t0 + c;
+            const bool mine = t < ntiles && sp[16 * tiles[t]] == p;
+            const unsigned long long m = __builtin_amdgcn_ballot_w64(mine);
+            if (lane == 0) cnt[s] = (int)__builtin_popcountll(m);
+            __syncthreads();
+            int at = nl;
+            for (int k = 0; k < MLP_WSUM_SPLIT; k++) {
+                at += k < s ? cnt[k] : 0;
+                nl += cnt[k];
+            }
+            if (mine) list[at + (int)__builtin_popcountll(m & ((1ull << lane) - 1ull))] = (unsigned short)t;
+            __syncthreads();
+        }
         if (c < MLP_TR_LOSS) {
             float acc = 0.f;
-            for (int t = 0; t < ntiles; t++)
-                if (mine[t]) acc += tpart[(size_t)t * MLP_TROW + c];
+#pragma unroll 4
+            for (int k = 0; k < nl; k++) acc += tpart[(size_t)list[k] * MLP_TROW + c];
             if (c < MLP_TR_B3)
-                grad[MLP_OFF_W3(np) + p * MLP_H + c] += acc;
+                put(&grad[MLP_OFF_W3(np) + p * MLP_H + c], acc);
             else if (c == MLP_TR_B3)
-                grad[MLP_OFF_B3(np) + p] += acc;
+                put(&grad[MLP_OFF_B3(np) + p], acc);
             else
-                gb1e[p * MLP_H + c - MLP_TR_B1E] += acc;
+                put(&gb1e[p * MLP_H + c - MLP_TR_B1E], acc);
         }
     } else {
-        float acc = 0.f;
-        for (int t = c; t < ntiles; t += 256) acc += tpart[(size_t)t * MLP_TROW + MLP_TR_LOSS];
-        red[c] = acc;
+        float *red = &part[0][0];
+        if (c < 256) {
+            float acc = 0.f;
+            for (int t = c; t < ntiles; t += 256) acc += tpart[(size_t)t * MLP_TROW + MLP_TR_LOSS];
+            red[c] = acc;
+        }
         __syncthreads();
         for (int w = 128; w > 0; w >>= 1) {
             if (c < w) red[c] += red[c + w];
@@ -378,11 +424,11 @@ __global__ __launch_bounds__(64 * MLP_WSUM_SPLIT) void k_mlp_chain(const float *
     acc = 0.f;
     for (int k = 0; k < MLP_WSUM_SPLIT; k++) acc += part[k][col];
     if (t < nb1)
-        grad[MLP_OFF_B1 + t] += acc;
+        grad[MLP_OFF_B1 + t] = 0.0f + acc;
     else if (t < nb1 + ne1)
-        grad[MLP_OFF_E1 + t - nb1] += acc;
+        grad[MLP_OFF_E1 + t - nb1] = 0.0f + acc;
     else
-        grad[MLP_OFF_EMB + t - nb1 - ne1] += acc;
+        grad[MLP_OFF_EMB + t - nb1 - ne1] = 0.0f + acc;
 }
 
 __global__ __launch_bounds__(256) void k_mlp_adam(float *__restrict__ theta, const float *__restrict__ grad,
@@ -703,25 +749,20 @@ struct mlp_bufs {
 };
 
 /* One gradient evaluation over the tiles tiles[0..ntiles) (device array) of
-   the samples (device arrays sr, sp, sE, sF): zero the gradients, then per
-   chunk of up to MLP_TCHUNK tiles k_mlp_grad, k_mlp_wsum and k_mlp_tsum,
-   then k_mlp_chain.  The mean loss adds into *B->loss. */
+   the samples (device arrays sr, sp, sE, sF): per chunk of up to MLP_TCHUNK
+   tiles k_mlp_grad and k_mlp_sums, then k_mlp_chain.  The mean loss adds into *B->loss. */
 static int mlp_gradient(struct gpu_state *g, const struct mlp_bufs *B, const float *sr, const int *sp,
                         const float *sE, const float *sF, const int *tiles, int ntiles, float wE, float wF) {
     const int np = g->mlp_np;
     const float inv_n = 1.0f / (16.0f * ntiles);
     if (ntiles < 1) return gerror_(engine_err_range, "empty batch");
-    hipLaunchKernelGGL(k_mlp_fill, dim3(64), dim3(256), 0, g->stream, B->grad, (long long)g->mlp_nparams, 0.0f);
-    hipLaunchKernelGGL(k_mlp_fill, dim3(16), dim3(256), 0, g->stream, B->gb1e, (long long)np * MLP_H, 0.0f);
     for (int c0 = 0; c0 < ntiles; c0 += MLP_TCHUNK) {
         const int nt = ntiles - c0 < MLP_TCHUNK ? ntiles - c0 : MLP_TCHUNK;
         const int grid = nt < B->grid_max ? nt : B->grid_max;
-        hipLaunchKernelGGL(k_mlp_grad, dim3(grid), dim3(64), 0, g->stream, gpu_mlp_net(g), sr, sp, sE, sF, tiles + c0,
-                           nt, wE, wF, inv_n, np, B->tpart, B->wpart, B->err);
-        hipLaunchKernelGGL(k_mlp_wsum, dim3((MLP_WPART + 63) / 64), dim3(64 * MLP_WSUM_SPLIT), 0, g->stream,
-                           B->wpart, grid, B->grad);
-        hipLaunchKernelGGL(k_mlp_tsum, dim3(np + 1), dim3(256), 0, g->stream, B->tpart, tiles + c0, nt, sp, np, B->grad,
-                           B->gb1e, B->loss, B->err);
+        hipLaunchKernelGGL(k_mlp_grad, dim3(grid), dim3(64 * MLP_GW), 0, g->stream, gpu_mlp_net(g), sr, sp, sE, sF,
+                           tiles + c0, nt, wE, wF, inv_n, np, B->tpart, B->wpart, B->err);
+        hipLaunchKernelGGL(k_mlp_sums, dim3(MLP_WBLOCKS + np + 1), dim3(64 * MLP_WSUM_SPLIT), 0, g->stream, B->wpart,
+                           grid, B->tpart, tiles + c0, nt, sp, np, c0 > 0, B->grad, B->gb1e, B->loss, B->err);
     }
     hipLaunchKernelGGL(k_mlp_chain, dim3((MLP_H + MLP_H * MLP_EMB + np * MLP_EMB + 63) / 64), dim3(64 * MLP_WSUM_SPLIT),
                        0, g->stream, g->d_theta, np, B->gb1e, B->grad);
