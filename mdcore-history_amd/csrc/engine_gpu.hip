@@ -1681,7 +1681,8 @@ __device__ __forceinline__ void block_tree3(double (*sd)[256], unsigned long lon
 __global__ __launch_bounds__(256) void k_reduce_one(int n, const double *__restrict__ acc,
                                                     const unsigned long long *__restrict__ cnt,
                                                     double *__restrict__ tot,
-                                                    unsigned long long *__restrict__ tot_cnt) {
+                                                    unsigned long long *__restrict__ tot_cnt,
+                                                    int *__restrict__ queue) {
     __shared__ double sd[3][256];
     __shared__ unsigned long long sc[3][256];
     const int t = threadIdx.x;
@@ -1707,6 +1708,7 @@ __global__ __launch_bounds__(256) void k_reduce_one(int n, const double *__restr
         tot[t] = sd[t][0];
         tot_cnt[t] = sc[t][0];
     }
+    if (t < MD_NQUEUE) queue[t] = 0; /* for the next pass */
 }
 
 __global__ __launch_bounds__(256) void k_reduce_a(int n, const double *__restrict__ acc,
@@ -1741,7 +1743,8 @@ __global__ __launch_bounds__(256) void k_reduce_a(int n, const double *__restric
 
 __global__ __launch_bounds__(256) void k_reduce_b(int nb, const double *__restrict__ pacc,
                                                   const unsigned long long *__restrict__ pcnt,
-                                                  double *__restrict__ tot, unsigned long long *__restrict__ tot_cnt) {
+                                                  double *__restrict__ tot, unsigned long long *__restrict__ tot_cnt,
+                                                  int *__restrict__ queue) {
     __shared__ double sd[3][256];
     __shared__ unsigned long long sc[3][256];
     const int t = threadIdx.x;
@@ -1760,6 +1763,7 @@ __global__ __launch_bounds__(256) void k_reduce_b(int nb, const double *__restri
         tot[t] = sd[t][0];
         tot_cnt[t] = sc[t][0];
     }
+    if (t < MD_NQUEUE) queue[t] = 0; /* for the next pass */
 }
 
 /* ------------------------------------------------------------ host side */
@@ -2631,12 +2635,12 @@ int gpu_launch(struct gpu_state *g, int timed, int mlp, int sort, int packed) {
     if (timed) HIPCHECK(hipEventRecord(g->ev[2], g->stream));
     if (nitems <= MD_RED_ONE)
         hipLaunchKernelGGL(k_reduce_one, dim3(1), dim3(256), 0, g->stream, nitems, g->d_cell_acc, g->d_cell_cnt,
-                           g->d_tot, g->d_tot_cnt);
+                           g->d_tot, g->d_tot_cnt, g->d_queue);
     else {
         hipLaunchKernelGGL(k_reduce_a, dim3(MD_RED_BLOCKS), dim3(256), 0, g->stream, nitems, g->d_cell_acc,
                            g->d_cell_cnt, g->d_red_acc, g->d_red_cnt);
         hipLaunchKernelGGL(k_reduce_b, dim3(1), dim3(256), 0, g->stream, MD_RED_BLOCKS, g->d_red_acc, g->d_red_cnt,
-                           g->d_tot, g->d_tot_cnt);
+                           g->d_tot, g->d_tot_cnt, g->d_queue);
     }
     if (timed) HIPCHECK(hipEventRecord(g->ev[3], g->stream));
     HIPCHECK(hipGetLastError());
