@@ -2,7 +2,8 @@
  * gfx950 nonbonded engine behind the mdcore C API (C-ABI in engine_gpu.h).
  *
  * One nonbonded pass is a chain of launches on one stream:
- *   k_pack      cell-ordered FP64 positions -> float4 (x, y, z, type bits),
+ *   k_pack      (at the upload, or with the migration of a resident step)
+ *               cell-ordered FP64 positions -> float4 (x, y, z, type bits),
  *               id -> slot map, slot -> cell map;
  *   k_sort_rank runner_dosort (runner_dosort.c:97-161) for every cell and
  *               every flagged direction: 16-bit projection keys computed in
@@ -214,20 +215,42 @@ __device__ __forceinline__ int rec_type(unsigned int w, int tshift) { return (in
 
 /* ------------------------------------------------------------ k_pack */
 
-__global__ __launch_bounds__(256) void k_pack(int nparts, const double *__restrict__ x, const int *__restrict__ type,
-                                              const int *__restrict__ id, int ncells,
-                                              const int *__restrict__ offset, float4 *__restrict__ xf,
+/* One wave per cell.  With dx, also the arrays of an upload from their one
+   staging block: with six copies, a cleared flag and the id clearing, the
+   device of a pass of 4,000 atoms was busy for 55 us before the sort; with one
+   copy and this kernel, and the clearing while the host packs, 12.  (The map
+   slot -> cell by a loop over the cell's slots in one thread: water, 125 atoms
+   per cell, 19 us; now 5.) */
+__global__ __launch_bounds__(256) void k_pack(int ncells, int nparts, const int2 *__restrict__ cnt_off,
+                                              const double *__restrict__ x, const int *__restrict__ type,
+                                              const int *__restrict__ id, float4 *__restrict__ xf,
                                               int *__restrict__ index_of_id, int *__restrict__ cell_of,
-                                              int *__restrict__ queue) {
-    int a = blockIdx.x * blockDim.x + threadIdx.x;
-    if (a == 0)
-        for (int q = 0; q < MD_NQUEUE; q++) queue[q] = 0;
-    if (a < nparts) {
-        xf[a] = make_float4((float)x[3 * a], (float)x[3 * a + 1], (float)x[3 * a + 2], __int_as_float(type[a]));
-        index_of_id[id[a]] = a;
+                                              double *__restrict__ dx, int *__restrict__ dtype, int *__restrict__ did,
+                                              int *__restrict__ dcount, int *__restrict__ doffset,
+                                              int2 *__restrict__ dcnt_off) {
+    const int c = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (c >= ncells) return;
+    const int2 co = cnt_off[c];
+    if (dx && lane == 0) {
+        dcount[c] = co.x;
+        doffset[c] = co.y;
+        dcnt_off[c] = co;
+        if (c == 0) doffset[ncells] = nparts;
     }
-    if (a < ncells)
-        for (int k = offset[a]; k < offset[a + 1]; k++) cell_of[k] = a;
+    for (int k = lane; k < co.x; k += 64) {
+        const int a = co.y + k, t = type[a], i = id[a];
+        const double x0 = x[3 * (size_t)a], x1 = x[3 * (size_t)a + 1], x2 = x[3 * (size_t)a + 2];
+        xf[a] = make_float4((float)x0, (float)x1, (float)x2, __int_as_float(t));
+        index_of_id[i] = a;
+        cell_of[a] = c;
+        if (dx) {
+            dx[3 * (size_t)a] = x0;
+            dx[3 * (size_t)a + 1] = x1;
+            dx[3 * (size_t)a + 2] = x2;
+            dtype[a] = t;
+            did[a] = i;
+        }
+    }
 }
 
 __global__ __launch_bounds__(256) void k_clear_ids(int nids, int *__restrict__ index_of_id) {
@@ -1682,6 +1705,8 @@ __global__ __launch_bounds__(256) void k_reduce_one(int n, const double *__restr
                                                     const unsigned long long *__restrict__ cnt,
                                                     double *__restrict__ tot,
                                                     unsigned long long *__restrict__ tot_cnt,
+                                                    double *__restrict__ htot,
+                                                    unsigned long long *__restrict__ htot_cnt,
                                                     int *__restrict__ queue) {
     __shared__ double sd[3][256];
     __shared__ unsigned long long sc[3][256];
@@ -1705,8 +1730,8 @@ __global__ __launch_bounds__(256) void k_reduce_one(int n, const double *__restr
     sc[2][t] = c2;
     block_tree3(sd, sc, t);
     if (t < 3) {
-        tot[t] = sd[t][0];
-        tot_cnt[t] = sc[t][0];
+        tot[t] = htot[t] = sd[t][0];
+        tot_cnt[t] = htot_cnt[t] = sc[t][0];
     }
     if (t < MD_NQUEUE) queue[t] = 0; /* for the next pass */
 }
@@ -1744,6 +1769,8 @@ __global__ __launch_bounds__(256) void k_reduce_a(int n, const double *__restric
 __global__ __launch_bounds__(256) void k_reduce_b(int nb, const double *__restrict__ pacc,
                                                   const unsigned long long *__restrict__ pcnt,
                                                   double *__restrict__ tot, unsigned long long *__restrict__ tot_cnt,
+                                                  double *__restrict__ htot,
+                                                  unsigned long long *__restrict__ htot_cnt,
                                                   int *__restrict__ queue) {
     __shared__ double sd[3][256];
     __shared__ unsigned long long sc[3][256];
@@ -1760,8 +1787,8 @@ __global__ __launch_bounds__(256) void k_reduce_b(int nb, const double *__restri
     }
     block_tree3(sd, sc, t);
     if (t < 3) {
-        tot[t] = sd[t][0];
-        tot_cnt[t] = sc[t][0];
+        tot[t] = htot[t] = sd[t][0];
+        tot_cnt[t] = htot_cnt[t] = sc[t][0];
     }
     if (t < MD_NQUEUE) queue[t] = 0; /* for the next pass */
 }
@@ -1777,14 +1804,11 @@ static void gpu_free_pass(struct gpu_state *g) {
     (void)hipFree(g->d_cell_of);
     (void)hipFree(g->d_xf);
     (void)hipFree(g->d_fhi);
-    (void)hipFree(g->d_flo);
+    (void)hipFree(g->d_stage);
     (void)hipFree(g->d_sortlist);
     (void)hipFree(g->d_keyof);
-    (void)hipHostFree(g->h_x);
-    (void)hipHostFree(g->h_type);
-    (void)hipHostFree(g->h_id);
+    (void)hipHostFree(g->h_stage);
     (void)hipHostFree(g->h_fhi);
-    (void)hipHostFree(g->h_flo);
     (void)hipHostFree(g->h_v);
     g->d_count = g->d_offset = NULL;
     g->d_x = NULL;
@@ -1792,8 +1816,10 @@ static void gpu_free_pass(struct gpu_state *g) {
     g->d_xf = g->d_fhi = g->d_flo = NULL;
     g->d_sortlist = NULL;
     g->d_keyof = NULL;
+    g->h_stage = g->d_stage = NULL;
     g->h_x = NULL;
     g->h_type = g->h_id = NULL;
+    g->h_cnt_off = NULL;
     g->h_fhi = g->h_flo = NULL;
     g->h_v = NULL;
     g->nparts_cap = 0;
@@ -1810,17 +1836,14 @@ static int gpu_alloc_parts(struct gpu_state *g, int n) {
     HIPCHECK(hipMalloc(&g->d_id, sizeof(int) * N));
     HIPCHECK(hipMalloc(&g->d_cell_of, sizeof(int) * N));
     HIPCHECK(hipMalloc(&g->d_xf, sizeof(float4) * N));
-    HIPCHECK(hipMalloc(&g->d_fhi, sizeof(float4) * N));
-    HIPCHECK(hipMalloc(&g->d_flo, sizeof(float4) * N));
+    HIPCHECK(hipMalloc(&g->d_fhi, sizeof(float4) * 2 * N)); /* and flo */
+    HIPCHECK(hipMalloc((void **)&g->d_stage, GPU_STAGE_BYTES(N, g->ncells)));
     HIPCHECK(hipMalloc(&g->d_sortlist, sizeof(unsigned int) * 13 * N));
     HIPCHECK(hipMalloc(&g->d_keyof, sizeof(unsigned short) * 13 * N));
     HIPCHECK(hipMalloc(&g->d_count, sizeof(int) * g->ncells));
     HIPCHECK(hipMalloc(&g->d_offset, sizeof(int) * (g->ncells + 1)));
-    HIPCHECK(hipHostMalloc((void **)&g->h_x, sizeof(double) * 3 * N, hipHostMallocDefault));
-    HIPCHECK(hipHostMalloc((void **)&g->h_type, sizeof(int) * N, hipHostMallocDefault));
-    HIPCHECK(hipHostMalloc((void **)&g->h_id, sizeof(int) * N, hipHostMallocDefault));
-    HIPCHECK(hipHostMalloc((void **)&g->h_fhi, sizeof(float4) * N, hipHostMallocDefault));
-    HIPCHECK(hipHostMalloc((void **)&g->h_flo, sizeof(float4) * N, hipHostMallocDefault));
+    HIPCHECK(hipHostMalloc((void **)&g->h_stage, GPU_STAGE_BYTES(N, g->ncells), hipHostMallocDefault));
+    HIPCHECK(hipHostMalloc((void **)&g->h_fhi, sizeof(float4) * 2 * N, hipHostMallocDefault)); /* and flo */
     HIPCHECK(hipHostMalloc((void **)&g->h_v, sizeof(double) * 3 * N, hipHostMallocDefault));
     g->nparts_cap = (int)N;
     return 0;
@@ -1897,9 +1920,9 @@ extern "C" int engine_gpu_finalize(struct engine *e) {
     (void)hipHostFree(g->h_cell_maxdx);
     free(g->h_sort_count);
     (void)hipHostFree(g->h_offset);
-    (void)hipHostFree(g->h_cnt_off);
     (void)hipHostFree(g->h_tot);
     (void)hipHostFree(g->h_tot_cnt);
+    (void)hipHostFree(g->h_flag);
     for (int k = 0; k < 8; k++) (void)hipEventDestroy(g->ev[k]);
     (void)hipStreamDestroy(g->stream);
     free(g);
@@ -2419,7 +2442,8 @@ extern "C" int engine_gpu_load(struct engine *e) {
     HIPCHECK(hipMalloc(&g->d_red_acc, sizeof(double) * 3 * MD_RED_BLOCKS));
     HIPCHECK(hipMalloc(&g->d_red_cnt, sizeof(unsigned long long) * 3 * MD_RED_BLOCKS));
     HIPCHECK(hipMalloc(&g->d_tot_cnt, sizeof(unsigned long long) * 4));
-    HIPCHECK(hipMalloc(&g->d_queue, sizeof(int) * (MD_NQUEUE + 1)));
+    HIPCHECK(hipMalloc(&g->d_queue, sizeof(int) * MD_NQUEUE));
+    HIPCHECK(hipMemset(g->d_queue, 0, sizeof(int) * MD_NQUEUE)); /* each pass leaves it zero */
     HIPCHECK(hipHostMalloc((void **)&g->h_count, sizeof(int) * s->nr_cells, hipHostMallocDefault));
     HIPCHECK(hipMalloc(&g->d_cell_maxdx, sizeof(double) * s->nr_cells));
     HIPCHECK(hipHostMalloc((void **)&g->h_cell_maxdx, sizeof(double) * s->nr_cells, hipHostMallocDefault));
@@ -2427,14 +2451,16 @@ extern "C" int engine_gpu_load(struct engine *e) {
         return gerror_(engine_err_malloc, "malloc failed");
     g->sort_valid = 0;
     HIPCHECK(hipHostMalloc((void **)&g->h_offset, sizeof(int) * (s->nr_cells + 1), hipHostMallocDefault));
-    HIPCHECK(hipHostMalloc((void **)&g->h_cnt_off, sizeof(int2) * s->nr_cells, hipHostMallocDefault));
+    HIPCHECK(hipHostMalloc((void **)&g->h_flag, sizeof(int), hipHostMallocDefault));
+    *g->h_flag = 0;
     HIPCHECK(hipHostMalloc((void **)&g->h_tot, sizeof(double) * 4, hipHostMallocDefault));
     HIPCHECK(hipHostMalloc((void **)&g->h_tot_cnt, sizeof(unsigned long long) * 4, hipHostMallocDefault));
 
     return engine_err_ok;
 }
 
-/* Pack host particles in cell order and upload them (no kernels). */
+/* Pack host particles in cell order and upload them; the device arrays of a
+   pass are those of the particles afterwards (gpu_launch: packed). */
 int gpu_upload(struct engine *e) {
     struct gpu_state *g = (struct gpu_state *)e->gpu;
     struct space *s = &e->s;
@@ -2448,6 +2474,15 @@ int gpu_upload(struct engine *e) {
         return gerror_(engine_err_maxparts, "more particles in a cell than the packed record holds (1024 for up to "
                                             "64 types, 256 for up to 256, 64 for up to 1024)");
     if (gpu_alloc_parts(g, n > 0 ? n : 1) < 0) return engine_err_gpu;
+    /* the id clearing runs while the host packs */
+    if (gpu_clear_ids(g) < 0) return engine_err_gpu;
+    /* one block: positions, types, ids, (count, offset) per cell */
+    g->h_x = (double *)g->h_stage;
+    g->h_type = (int *)(g->h_x + 3 * (size_t)n);
+    g->h_id = g->h_type + n;
+    g->h_cnt_off = (int2 *)(g->h_id + n);
+    g->d_flo = g->d_fhi + n;
+    g->h_flo = g->h_fhi + n;
     if (space_pack(s, g->max_type, g->h_count, g->h_offset, (int *)g->h_cnt_off, g->h_x, g->h_type, g->h_id, &maxc,
                    &maxid) < 0)
         return gerror_(engine_err_range, "particle type out of range");
@@ -2468,14 +2503,15 @@ int gpu_upload(struct engine *e) {
     g->P.nparts = n;
     g->P.nids = g->nids;
     g->P.maxn = maxc > 0 ? maxc : 1;
-    HIPCHECK(hipMemcpyAsync(g->d_x, g->h_x, sizeof(double) * 3 * n, hipMemcpyHostToDevice, g->stream));
-    HIPCHECK(hipMemcpyAsync(g->d_type, g->h_type, sizeof(int) * n, hipMemcpyHostToDevice, g->stream));
-    HIPCHECK(hipMemcpyAsync(g->d_id, g->h_id, sizeof(int) * n, hipMemcpyHostToDevice, g->stream));
-    HIPCHECK(hipMemcpyAsync(g->d_count, g->h_count, sizeof(int) * s->nr_cells, hipMemcpyHostToDevice, g->stream));
-    HIPCHECK(hipMemcpyAsync(g->d_offset, g->h_offset, sizeof(int) * (s->nr_cells + 1), hipMemcpyHostToDevice,
-                            g->stream));
-    HIPCHECK(hipMemcpyAsync(g->d_cnt_off, g->h_cnt_off, sizeof(int2) * s->nr_cells, hipMemcpyHostToDevice,
-                            g->stream));
+    HIPCHECK(hipMemcpyAsync(g->d_stage, g->h_stage, GPU_STAGE_BYTES(n, s->nr_cells), hipMemcpyHostToDevice, g->stream));
+    {
+        const double *x = (const double *)g->d_stage;
+        const int *type = (const int *)(x + 3 * (size_t)n), *id = type + n;
+        hipLaunchKernelGGL(k_pack, dim3((s->nr_cells + 3) / 4), dim3(256), 0, g->stream, s->nr_cells, n,
+                           (const int2 *)(id + n), x, type, id, g->d_xf, g->d_index_of_id, g->d_cell_of, g->d_x,
+                           g->d_type, g->d_id, g->d_count, g->d_offset, g->d_cnt_off);
+        HIPCHECK(hipGetLastError());
+    }
     return engine_err_ok;
 }
 
@@ -2488,7 +2524,7 @@ int gpu_clear_ids(struct gpu_state *g) {
 }
 
 /* Launch the kernels of one pass on the resident particles, with events
-   around each when timed; mlp selects the surrogate mode of the pair kernel.
+   around each when timed (2: around the whole); mlp selects the surrogate mode of the pair kernel.
    sort: 0 keeps the keys and sort lists of the last sort; packed: d_xf and
    the id and cell maps are those of the particles already. */
 int gpu_launch(struct gpu_state *g, int timed, int mlp, int sort, int packed) {
@@ -2567,10 +2603,10 @@ int gpu_launch(struct gpu_state *g, int timed, int mlp, int sort, int packed) {
 
     if (timed) HIPCHECK(hipEventRecord(g->ev[0], g->stream));
     if (!packed && gpu_clear_ids(g) < 0) return engine_err_gpu;
-    nb = ((g->nparts > g->ncells ? g->nparts : g->ncells) + 255) / 256;
     if (!packed)
-        hipLaunchKernelGGL(k_pack, dim3(nb), dim3(256), 0, g->stream, g->nparts, g->d_x, g->d_type, g->d_id, g->ncells,
-                       g->d_offset, g->d_xf, g->d_index_of_id, g->d_cell_of, g->d_queue);
+        hipLaunchKernelGGL(k_pack, dim3((g->ncells + 3) / 4), dim3(256), 0, g->stream, g->ncells, g->nparts,
+                           g->d_cnt_off, g->d_x, g->d_type, g->d_id, g->d_xf, g->d_index_of_id, g->d_cell_of,
+                           (double *)NULL, (int *)NULL, (int *)NULL, (int *)NULL, (int *)NULL, (int2 *)NULL);
     if (!sort) {
         /* pseudo-Verlet step between rebuilds: the keys and sort lists of
            the last sort stay (runner.c:773) */
@@ -2582,15 +2618,15 @@ int gpu_launch(struct gpu_state *g, int timed, int mlp, int sort, int packed) {
            few cells one wave per direction */
         const int bs = maxn > MD_SORT_ONEWAVE_MAX || g->ncells <= MD_SORT_FEW ? 13 * 64 : 64;
         hipLaunchKernelGGL(k_sort_rank, dim3(g->ncells), dim3(bs), sh, g->stream, P, g->d_count, g->d_offset,
-                           g->d_sortflags, g->d_x, g->d_sortlist, g->d_keyof, g->d_kminmax, g->d_queue + MD_NQUEUE,
+                           g->d_sortflags, g->d_x, g->d_sortlist, g->d_keyof, g->d_kminmax, g->h_flag,
                            maxn);
     } else {
         nb = (g->ncells * 13 + 255) / 256;
         hipLaunchKernelGGL(k_sort, dim3(nb), dim3(256), 0, g->stream, P, g->d_count, g->d_offset, g->d_sortflags,
-                           g->d_x, g->d_sortlist, g->d_keyof, g->d_kminmax, g->d_queue + MD_NQUEUE);
+                           g->d_x, g->d_sortlist, g->d_keyof, g->d_kminmax, g->h_flag);
     }
     if (sort) g->sort_valid = 1;
-    if (timed) HIPCHECK(hipEventRecord(g->ev[1], g->stream));
+    if (timed == 1) HIPCHECK(hipEventRecord(g->ev[1], g->stream));
     struct nb_out O;
     O.fhi = g->d_fhi;
     O.flo = g->d_flo;
@@ -2632,15 +2668,15 @@ int gpu_launch(struct gpu_state *g, int timed, int mlp, int sort, int packed) {
         hipLaunchKernelGGL(k_fold, dim3(g->ncells), dim3(64), 0, g->stream, g->ncells, g->d_cnt_off, nsplit,
                            g->nparts, (const float4 *)g->d_phi, (const float4 *)g->d_plo, half,
                            g->d_inv_off, g->d_inv_cell, g->d_jpart, g->d_fhi, g->d_flo);
-    if (timed) HIPCHECK(hipEventRecord(g->ev[2], g->stream));
+    if (timed == 1) HIPCHECK(hipEventRecord(g->ev[2], g->stream));
     if (nitems <= MD_RED_ONE)
         hipLaunchKernelGGL(k_reduce_one, dim3(1), dim3(256), 0, g->stream, nitems, g->d_cell_acc, g->d_cell_cnt,
-                           g->d_tot, g->d_tot_cnt, g->d_queue);
+                           g->d_tot, g->d_tot_cnt, g->h_tot, g->h_tot_cnt, g->d_queue);
     else {
         hipLaunchKernelGGL(k_reduce_a, dim3(MD_RED_BLOCKS), dim3(256), 0, g->stream, nitems, g->d_cell_acc,
                            g->d_cell_cnt, g->d_red_acc, g->d_red_cnt);
         hipLaunchKernelGGL(k_reduce_b, dim3(1), dim3(256), 0, g->stream, MD_RED_BLOCKS, g->d_red_acc, g->d_red_cnt,
-                           g->d_tot, g->d_tot_cnt, g->d_queue);
+                           g->d_tot, g->d_tot_cnt, g->h_tot, g->h_tot_cnt, g->d_queue);
     }
     if (timed) HIPCHECK(hipEventRecord(g->ev[3], g->stream));
     HIPCHECK(hipGetLastError());
@@ -2679,8 +2715,7 @@ extern "C" int engine_gpu_sync(struct engine *e, unsigned int what) {
         free(tmp);
     }
     if (what & engine_gpu_sync_forces_down) {
-        HIPCHECK(hipMemcpyAsync(g->h_fhi, g->d_fhi, sizeof(float4) * g->nparts, hipMemcpyDeviceToHost, g->stream));
-        HIPCHECK(hipMemcpyAsync(g->h_flo, g->d_flo, sizeof(float4) * g->nparts, hipMemcpyDeviceToHost, g->stream));
+        HIPCHECK(hipMemcpyAsync(g->h_fhi, g->d_fhi, sizeof(float4) * 2 * g->nparts, hipMemcpyDeviceToHost, g->stream));
         HIPCHECK(hipMemcpyAsync(g->h_tot, g->d_tot, sizeof(double) * 3, hipMemcpyDeviceToHost, g->stream));
         HIPCHECK(hipMemcpyAsync(g->h_tot_cnt, g->d_tot_cnt, sizeof(unsigned long long) * 3, hipMemcpyDeviceToHost,
                                 g->stream));
@@ -2729,7 +2764,6 @@ static void gpu_sorted(struct engine *e, struct gpu_state *g) {
 extern "C" int engine_nonbond_gpu(struct engine *e) {
     struct gpu_state *g;
     struct space *s;
-    int flag = 0;
     if (e == NULL) return gerror_(engine_err_null, "NULL engine");
     g = (struct gpu_state *)e->gpu;
     if (g == NULL) return gerror_(engine_err_nogpu, "engine_gpu_load was not called");
@@ -2740,17 +2774,12 @@ extern "C" int engine_nonbond_gpu(struct engine *e) {
     e->timers[engine_timer_gpu_load] = gpu_wall() - tw;
     int sort = 1;
     if (gpu_verlet(e, g, &sort) < 0) return engine_err_range;
-    HIPCHECK(hipMemsetAsync(g->d_queue + MD_NQUEUE, 0, sizeof(int), g->stream));
-    if (gpu_launch(g, 1, (e->flags & engine_flag_mlp) != 0, sort, 0) < 0) return engine_err_gpu;
-    if (sort) gpu_sorted(e, g);
-    HIPCHECK(hipMemcpyAsync(g->h_fhi, g->d_fhi, sizeof(float4) * g->nparts, hipMemcpyDeviceToHost, g->stream));
-    HIPCHECK(hipMemcpyAsync(g->h_flo, g->d_flo, sizeof(float4) * g->nparts, hipMemcpyDeviceToHost, g->stream));
-    HIPCHECK(hipMemcpyAsync(g->h_tot, g->d_tot, sizeof(double) * 3, hipMemcpyDeviceToHost, g->stream));
-    HIPCHECK(hipMemcpyAsync(g->h_tot_cnt, g->d_tot_cnt, sizeof(unsigned long long) * 3, hipMemcpyDeviceToHost,
-                            g->stream));
-    HIPCHECK(hipMemcpyAsync(&flag, g->d_queue + MD_NQUEUE, sizeof(int), hipMemcpyDeviceToHost, g->stream));
+    *g->h_flag = 0; /* nothing is under way that could set it */
+    if (gpu_launch(g, 2, (e->flags & engine_flag_mlp) != 0, sort, 1) < 0) return engine_err_gpu;
+    HIPCHECK(hipMemcpyAsync(g->h_fhi, g->d_fhi, sizeof(float4) * 2 * g->nparts, hipMemcpyDeviceToHost, g->stream));
+    if (sort) gpu_sorted(e, g); /* meanwhile */
     HIPCHECK(hipStreamSynchronize(g->stream));
-    if (flag) return gerror_(engine_err_range, "sort stack overflow");
+    if (*(const volatile int *)g->h_flag) return gerror_(engine_err_range, "sort stack overflow");
     {
         float ms = 0.0f;
         HIPCHECK(hipEventElapsedTime(&ms, g->ev[0], g->ev[3]));

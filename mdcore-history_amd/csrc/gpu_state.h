@@ -17,6 +17,8 @@
 #define MD_SORT_LDS_MAX 480    /* k_sort_rank's cells: 63.5 KiB of LDS at 480 */
 #define MD_SORT_ONEWAVE_MAX 64 /* those of them that one wave sorts */
 
+#define GPU_STAGE_BYTES(n, nc) (32 * (size_t)(n) + 8 * (size_t)(nc))
+
 #define gerror_(id, msg) errs_register((id), (msg), __LINE__, __func__, __FILE__)
 
 #define HIPCHECK(call)                                                                            \
@@ -115,7 +117,11 @@ struct gpu_state {
     double *d_cell_maxdx, *h_cell_maxdx;
     int sort_valid;
     int *h_sort_count;
-    /* pinned host staging */
+    /* pinned host staging: the block of an upload (x, type, id, (count,
+       offset) of the uploaded particles, one after the other) and its copy on
+       the device; flo follows fhi in the same block */
+    char *h_stage, *d_stage;
+    int *h_flag; /* pinned: set by a sort that overflows */
     double *h_x;
     int *h_type, *h_id, *h_count, *h_offset;
     int2 *h_cnt_off;

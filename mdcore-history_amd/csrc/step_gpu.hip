@@ -345,10 +345,9 @@ __global__ __launch_bounds__(256) void k_settle(struct step_geom G, const int *_
                                                 double *__restrict__ v2, int *__restrict__ id2,
                                                 int *__restrict__ type2, int *__restrict__ st, int pack,
                                                 float4 *__restrict__ xf, int *__restrict__ index_of_id,
-                                                int *__restrict__ cell_of, int *__restrict__ queue) {
+                                                int *__restrict__ cell_of) {
 #pragma clang fp contract(off)
     const int c = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (pack && blockIdx.x == 0 && threadIdx.x < MD_NQUEUE) queue[threadIdx.x] = 0;
     if (c >= G.ncells) return;
     auto put = [&](int a, int b, const double *xn) {
         const int i = id[a], t = type[a];
@@ -852,7 +851,7 @@ static int step_migrate(struct gpu_state *g, struct step_bufs *b, const struct s
     }
     hipLaunchKernelGGL(k_settle, dim3((nc + 3) / 4), dim3(256), 0, g->stream, G, g->d_count, g->d_offset, b->slot,
                        b->ndep, b->qsrc, b->qdest, b->offset2, b->stay, g->d_x, b->v, g->d_id, g->d_type, b->x2, b->v2,
-                       b->id2, b->type2, b->st, pack, g->d_xf, g->d_index_of_id, g->d_cell_of, g->d_queue);
+                       b->id2, b->type2, b->st, pack, g->d_xf, g->d_index_of_id, g->d_cell_of);
     HIPCHECK(hipEventRecord(g->ev[4], g->stream));
     HIPCHECK(hipGetLastError());
     double *t;
@@ -905,11 +904,7 @@ static int step_download(struct engine *e, struct gpu_state *g, struct step_bufs
         hipMemcpyAsync(count, g->d_count, sizeof(int) * nc, hipMemcpyDeviceToHost, g->stream) != hipSuccess ||
         hipMemcpyAsync(ioi, g->d_index_of_id, sizeof(int) * g->nids, hipMemcpyDeviceToHost, g->stream) != hipSuccess ||
         hipMemcpyAsync(es, b->esteps, sizeof(double) * 4 * nsteps, hipMemcpyDeviceToHost, g->stream) != hipSuccess ||
-        hipMemcpyAsync(g->h_fhi, g->d_fhi, sizeof(float4) * n, hipMemcpyDeviceToHost, g->stream) != hipSuccess ||
-        hipMemcpyAsync(g->h_flo, g->d_flo, sizeof(float4) * n, hipMemcpyDeviceToHost, g->stream) != hipSuccess ||
-        hipMemcpyAsync(g->h_tot, g->d_tot, sizeof(double) * 3, hipMemcpyDeviceToHost, g->stream) != hipSuccess ||
-        hipMemcpyAsync(g->h_tot_cnt, g->d_tot_cnt, sizeof(unsigned long long) * 3, hipMemcpyDeviceToHost,
-                       g->stream) != hipSuccess ||
+        hipMemcpyAsync(g->h_fhi, g->d_fhi, sizeof(float4) * 2 * n, hipMemcpyDeviceToHost, g->stream) != hipSuccess ||
         (verlet && (hipMemcpyAsync(ox, b->oldx, sizeof(double) * 3 * n, hipMemcpyDeviceToHost, g->stream) != hipSuccess ||
                     hipMemcpyAsync(cm, g->d_cell_maxdx, sizeof(double) * nc, hipMemcpyDeviceToHost, g->stream) !=
                         hipSuccess)) ||
@@ -1152,7 +1147,7 @@ static int steps_verlet(struct engine *e, struct gpu_state *g, struct step_bufs 
     }
     /* whether the pass's FP32 positions and maps are those of the current
        particles; whether this step's pass is already under way */
-    int packed = 0, under = 0;
+    int packed = 1, under = 0;
     for (int step = 0; step < nsteps; step++) {
         if (!rebuild) {
             /* engine_verlet_update without a pending rebuild */
@@ -1209,7 +1204,7 @@ extern "C" int engine_gpu_steps(struct engine *e, int nsteps, double *epot, doub
     struct space *s;
     struct step_bufs b;
     struct step_geom G;
-    int rc = engine_err_ok, maxc = 0, outside = 0, flag = 0;
+    int rc = engine_err_ok, maxc = 0, outside = 0;
     if (e == NULL) return gerror_(engine_err_null, "NULL engine");
     g = (struct gpu_state *)e->gpu;
     if (g == NULL) return gerror_(engine_err_nogpu, "engine_gpu_load was not called");
@@ -1217,6 +1212,7 @@ extern "C" int engine_gpu_steps(struct engine *e, int nsteps, double *epot, doub
     if (nsteps == 0) return engine_err_ok;
     s = &e->s;
     HIPCHECK(hipSetDevice(g->device));
+    *g->h_flag = 0;
     if (gpu_upload(e) < 0) return engine_err_gpu;
     for (int k = 0; k < 3; k++) {
         G.h[k] = s->h[k];
@@ -1240,8 +1236,7 @@ extern "C" int engine_gpu_steps(struct engine *e, int nsteps, double *epot, doub
             space_pack_v(s, g->h_offset, v);
             if (hipMemcpy(b.mass, mass, sizeof(double) * g->max_type, hipMemcpyHostToDevice) != hipSuccess ||
                 hipMemcpy(b.imass, imass, sizeof(double) * g->max_type, hipMemcpyHostToDevice) != hipSuccess ||
-                hipMemcpyAsync(b.v, v, sizeof(double) * 3 * g->nparts, hipMemcpyHostToDevice, g->stream) != hipSuccess ||
-                hipMemsetAsync(g->d_queue + MD_NQUEUE, 0, sizeof(int), g->stream) != hipSuccess)
+                hipMemcpyAsync(b.v, v, sizeof(double) * 3 * g->nparts, hipMemcpyHostToDevice, g->stream) != hipSuccess)
                 rc = gerror_(engine_err_gpu, "upload failed");
         }
         free(mass);
@@ -1250,7 +1245,6 @@ extern "C" int engine_gpu_steps(struct engine *e, int nsteps, double *epot, doub
     const int verlet = (e->flags & engine_flag_verlet) != 0;
     double smaxdx = s->maxdx;
     if (rc == engine_err_ok) rc = rigid_upload(e, g, &b);
-    if (rc == engine_err_ok && gpu_clear_ids(g) < 0) rc = engine_err_gpu;
     if (verlet && rc == engine_err_ok)
         rc = steps_verlet(e, g, &b, G, nsteps, &smaxdx);
     /* engine_step: shuffle, pass, advance.  After an advance that left every
@@ -1292,11 +1286,9 @@ extern "C" int engine_gpu_steps(struct engine *e, int nsteps, double *epot, doub
         g->maxcount = maxc;
         g->P.maxn = maxc > 0 ? maxc : 1;
     }
-    if (rc == engine_err_ok &&
-        (hipMemcpyAsync(&flag, g->d_queue + MD_NQUEUE, sizeof(int), hipMemcpyDeviceToHost, g->stream) != hipSuccess ||
-         hipStreamSynchronize(g->stream) != hipSuccess))
+    if (rc == engine_err_ok && hipStreamSynchronize(g->stream) != hipSuccess)
         rc = gerror_(engine_err_gpu, "step failed");
-    if (rc == engine_err_ok && flag) rc = gerror_(engine_err_range, "sort stack overflow");
+    if (rc == engine_err_ok && *(const volatile int *)g->h_flag) rc = gerror_(engine_err_range, "sort stack overflow");
     if (rc == engine_err_ok) rc = step_download(e, g, &b, nsteps, epot, ekin, verlet, smaxdx);
     (void)hipStreamSynchronize(g->stream);
     step_free_rigid(&b);
