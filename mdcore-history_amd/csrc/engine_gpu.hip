@@ -1597,10 +1597,19 @@ __device__ __forceinline__ void nonbond_body(
     P, cnt_off, nbr, nbr_off, nbr_mid, nbs, origin, loc, xf, x64, pid, kminmax, sortlist, keyof, ptab, \
         coeffs4, excl_off, excl_list, index_of_id, cell_of, O
 
-template <int R, bool PROJ>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(R == 32 ? 4 : 3, 8))) void k_pair(PAIR_PARAMS) {
-    __shared__ __attribute__((aligned(16))) pair_lds<R> L;
-    pair_body<R, PROJ>(L, PAIR_ARGS);
+template <int R, int TABS, bool PROJ>
+__global__ __launch_bounds__(64 * PT_WAVES) __attribute__((amdgpu_waves_per_eu(R == 32 ? 4 : 3, 8))) void k_pair(
+    PAIR_PARAMS) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    /* the waves' working sets, then the tables */
+    pair_lds<R> *L = (pair_lds<R> *)smem;
+    float4 *tab = (float4 *)(L + PT_WAVES);
+    if (TABS) {
+        const int nh = P.ptab_bytes / 16, nt = nh + (TABS == 2 ? P.coef_bytes / 16 : 0);
+        for (int k = threadIdx.x; k < nt; k += 64 * PT_WAVES) tab[k] = k < nh ? ptab[k] : coeffs4[k - nh];
+        __syncthreads();
+    }
+    pair_body<R, TABS, PROJ>(L[threadIdx.x >> 6], (const char *)tab, PAIR_ARGS);
 }
 
 /* Surrogate mode (engine_flag_mlp). */
@@ -2637,11 +2646,25 @@ int gpu_launch(struct gpu_state *g, int timed, int mlp, int sort, int packed) {
     O.plo = g->d_plo;
     const int nitems = g->ncells * nsplit;
     if (pair) {
-        static const decltype(&k_pair<32, false>) kp[2][2] = {{k_pair<32, false>, k_pair<32, true>},
-                                                              {k_pair<64, false>, k_pair<64, true>}};
+        static const decltype(&k_pair<32, 0, false>) kp[2][3][2] = {
+            {{k_pair<32, 0, false>, k_pair<32, 0, true>},
+             {k_pair<32, 1, false>, k_pair<32, 1, true>},
+             {k_pair<32, 2, false>, k_pair<32, 2, true>}},
+            {{k_pair<64, 0, false>, k_pair<64, 0, true>},
+             {k_pair<64, 1, false>, k_pair<64, 1, true>},
+             {k_pair<64, 2, false>, k_pair<64, 2, true>}}};
+        /* the tables in LDS as far as PT_TAB bytes hold them: with them 4
+           blocks of 4 waves still fit on a CU, and every access kept from the
+           L1 counts (argon 864,000 atoms, all in LDS: 622 -> 595 us; 20 types,
+           the headers: 4180 -> 3670 us) */
+        const int tabs = P.ptab_bytes + P.coef_bytes <= PT_TAB ? 2 : P.ptab_bytes <= PT_TAB ? 1 : 0;
+        const size_t plds = PT_WAVES * (big ? sizeof(pair_lds<64>) : sizeof(pair_lds<32>)) +
+                            (tabs ? P.ptab_bytes : 0) + (tabs == 2 ? P.coef_bytes : 0);
         /* the same number of blocks for each die */
-        const dim3 grid((nitems + MD_NQUEUE - 1) / MD_NQUEUE * MD_NQUEUE);
-        hipLaunchKernelGGL(kp[big][P.proj != 0], grid, dim3(64), 0, g->stream, P, g->d_cnt_off, g->d_nbr, g->d_nbr_off,
+        const int nblocks = (nitems + PT_WAVES - 1) / PT_WAVES;
+        const dim3 grid((nblocks + MD_NQUEUE - 1) / MD_NQUEUE * MD_NQUEUE);
+        hipLaunchKernelGGL(kp[big][tabs][P.proj != 0], grid, dim3(64 * PT_WAVES), plds, g->stream, P, g->d_cnt_off,
+                           g->d_nbr, g->d_nbr_off,
                            g->d_nbr_mid, g->d_nbs, g->d_origin, g->d_loc, g->d_xf, g->d_x, g->d_id,
                            g->d_kminmax, g->d_sortlist, g->d_keyof, g->d_ptab, (const float4 *)g->d_coeffs,
                            g->d_excl_off, g->d_excl_list, g->d_index_of_id, g->d_cell_of, O);

@@ -44,28 +44,34 @@
  * key_j + dnshift - key_i <= dscale (x_j + shift - x_i).n + 1 <= dscale rc + 1
  * < dmaxdist for every pair within the cutoff.
  *
- * What bounds it: VALU issue (about 60 % busy), 71 instructions per hit and
- * lane on the i side at half the lanes busy (an atom's hits per chunk differ),
- * 60 on the j side at 97 %; with 20 types also the coefficients, 384 KB of
- * tables read at random through the 32 KB L1 (0.8 lines from L2 per hit).
+ * What bounds it: VALU issue (85 % busy on 20 types), 71 instructions per hit
+ * and lane on the i side at half the lanes busy (an atom's hits per chunk
+ * differ), 60 on the j side at 97 %; with 20 types the coefficients come next,
+ * 384 KB of tables read at random through the 32 KB L1.  The L1 serves about a
+ * lane a clock, so a lane without a hit asks for nothing (mixture 1,048,576:
+ * 3.0e9 accesses, 1.2 a clock, 4360 us; without them 2.3e9, 4180), and the
+ * table headers lie in LDS (1.6e9, 3670), copied once per PT_WAVES waves.
  * The filter costs 5/256 VALU instructions per candidate, against 27/64 at
  * 45 % lane use for the walk along the sorted windows that it replaced.
- * Kernel time with that walk and now, us: mixture 1,048,576 atoms 4695, 4360;
- * 99,991 atoms 929, 480; 4,000 atoms 618, 115; argon 1,048,576 atoms 1290,
- * 740; 32,000 atoms 190, 53; 4,000 atoms 82, 27; water 64,000 atoms 555, 330.
- * Also measured, mixture 1,048,576: both sides dealt evenly (3350 us, but the
- * energies' FP32 sums then run in another order, up to 2e-6 of the total off
- * where it cancels); the j hits levelling the i lanes in one loop 5180; chunks
- * of 192 slots 4570 (12 waves per CU instead of 16); 3 waves per SIMD 4950;
- * tables in LDS, two lanes fetching each 32-byte row together: within 4 %.
+ * Kernel time with that walk and now, us: mixture 1,048,576 atoms 4695, 3670;
+ * 99,991 atoms 929, 440; 4,000 atoms 618, 114; argon 1,048,576 atoms 1290,
+ * 720; 32,000 atoms 190, 53; 4,000 atoms 82, 28; water 64,000 atoms 555, 327.
+ * Also measured, mixture 1,048,576, before the headers lay in LDS: both sides
+ * dealt evenly (3350 us, but the energies' FP32 sums then run in another
+ * order, up to 2e-6 of the total off where it cancels); the j hits levelling
+ * the i lanes in one loop 5180; chunks of 192 slots 4570 (12 waves per CU
+ * instead of 16); 3 waves per SIMD 4950; two lanes fetching each 32-byte row
+ * together: within 4 %.
  */
 #ifndef PAIR_TILE_H
 #define PAIR_TILE_H
 
 #define PT_TC 128    /* slots per chunk, a multiple of 64 */
 #define PT_FSLOT 64  /* j side: sums of owner atoms in pair_lds::F, after those of the 64 runs */
-#define PT_NPP 24    /* i side: pieces (16 slots of one entry at most) dealt at a time */
-#define PT_LS 26     /* i side: half words of a lane's list; 13 words, so that lanes differ in bank */
+#define PT_NPP 16    /* i side: pieces (16 slots of one entry at most) dealt at a time */
+#define PT_LS 18     /* i side: half words of a lane's list; 9 words, so that lanes differ in bank */
+#define PT_WAVES 4   /* items per block: they share the LDS copy of the tables */
+#define PT_TAB 8192  /* bytes of LDS for table headers and coefficients */
 
 typedef float pt_f4 __attribute__((ext_vector_type(4)));
 
@@ -79,7 +85,7 @@ struct pair_lds {
     float4 S[PT_TC];          /* x, y, z in the owner's frame; type | entry << 10 | key << 16    */
     float4 own[R];            /* x, y, z, byte offset of the type's table-header row             */
     int2 E[64];               /* per entry: first slot | sid << 17 | count << 21, cell offset    */
-    int2 W[64];               /* per entry: dmaxdist - dnshift; own_key row | sign               */
+    int W[64];                /* per entry: dmaxdist - dnshift                                   */
     unsigned short okey[13 * R];
     union {
         float Q[PT_TC]; /* |x|^2 for the filter                                                  */
@@ -125,10 +131,12 @@ __device__ __forceinline__ float pt_offset(float r2, float ir, float c) {
     return r - c;
 }
 
-/* PROJ: the projected window (every pair within the cutoff); the pass also
+/* TABS: 1, 2: the table headers (and 2: the coefficients) are in LDS at tab.
+   PROJ: the projected window (every pair within the cutoff); the pass also
    counts the pairs that the reference window admits. */
-template <int R, bool PROJ>
-__device__ __forceinline__ void pair_body(pair_lds<R> &L, const struct nb_params &P, const int2 *__restrict__ cnt_off,
+template <int R, int TABS, bool PROJ>
+__device__ __forceinline__ void pair_body(pair_lds<R> &L, const char *tab, const struct nb_params &P,
+                                          const int2 *__restrict__ cnt_off,
                                           const int4 *__restrict__ nbr, const int *__restrict__ nbr_off,
                                           const int *__restrict__ nbr_mid, const float4 *__restrict__ nbs,
                                           const double *__restrict__ origin,
@@ -142,7 +150,7 @@ __device__ __forceinline__ void pair_body(pair_lds<R> &L, const struct nb_params
                                           const int *__restrict__ cell_of, const struct nb_out &O) {
     typedef pair_lds<R> pair_lds_t;
     constexpr int NIT = R / 16, KW = (R * PT_TC / 32 + 63) / 64;
-    const int lane = threadIdx.x, ln = lane & 15, g = lane >> 4;
+    const int lane = threadIdx.x & 63, ln = lane & 15, g = lane >> 4;
     const int mt = P.max_type;
     unsigned int *const raw = (unsigned int *)L.wl;
     unsigned short *const lst = L.lst + lane * PT_LS;
@@ -155,12 +163,13 @@ __device__ __forceinline__ void pair_body(pair_lds<R> &L, const struct nb_params
     const __amdgpu_buffer_rsrc_t rs_ptab = make_rsrc(ptab, P.ptab_bytes);
     const __amdgpu_buffer_rsrc_t rs_coef = make_rsrc(coeffs4, P.coef_bytes);
 
-    /* One item per block (one wave): (owner cell, neighbour group).  Blocks
-       go to the 8 compute dies in turn, so block b takes the (b / 8)-th item
-       of die b % 8's contiguous share of the work order. */
+    /* One item per wave: (owner cell, neighbour group).  Blocks go to the 8
+       compute dies in turn, so block b takes the (b / 8)-th block of die
+       b % 8's contiguous share of the work order. */
     const int nitems = P.ncells * P.nsplit;
-    const int item =
-        ((int)blockIdx.x % MD_NQUEUE) * ((int)gridDim.x / MD_NQUEUE) + (int)blockIdx.x / MD_NQUEUE;
+    const int item = __builtin_amdgcn_readfirstlane(
+        (((int)blockIdx.x % MD_NQUEUE) * ((int)gridDim.x / MD_NQUEUE) + (int)blockIdx.x / MD_NQUEUE) * PT_WAVES +
+        (int)(threadIdx.x >> 6));
     if (item >= nitems) return;
     const int ci = item / P.nsplit, grp = item - ci * P.nsplit;
     const int c = P.order[ci];
@@ -269,7 +278,7 @@ __device__ __forceinline__ void pair_body(pair_lds<R> &L, const struct nb_params
             if (total == 0) continue;
             wave_lds_sync();
             L.E[lane] = make_int2((int)((unsigned int)pex | ((unsigned int)esid << 17) | ((unsigned int)ecnt << 21)), eoff);
-            L.W[lane] = make_int2(wcst, (esid * R) | (side ? 1 << 31 : 0));
+            L.W[lane] = wcst;
             /* the self task's entry, if any, and its first slot */
             const unsigned long long selfm = __builtin_amdgcn_ballot_w64(eself && len > 0);
             const int eslf = selfm ? (int)__builtin_ctzll(selfm) : -1;
@@ -417,8 +426,11 @@ __device__ __forceinline__ void pair_body(pair_lds<R> &L, const struct nb_params
                     cur &= cur - 1u;
                     const float4 pj = *(const float4 *)((const char *)L.S + tb + 16 * bit);
                     const unsigned int w = __float_as_uint(pj.w);
+                    /* a lane without a hit loads nothing (past the end): half
+                       the lanes on the i side, and the L1 serves a lane a
+                       clock */
                     const int ho = __float_as_int(xi.w) + 16 * (int)__builtin_amdgcn_ubfe(w, 0, 10);
-                    const float4 hd = ld_f4(rs_ptab, ho);
+                    const float4 hd = TABS ? *(const float4 *)(tab + (have ? ho : 0)) : ld_f4(rs_ptab, have ? ho : -16);
                     v.dx = xi.x - pj.x;
                     v.dy = xi.y - pj.y;
                     v.dz = xi.z - pj.z;
@@ -435,11 +447,10 @@ __device__ __forceinline__ void pair_body(pair_lds<R> &L, const struct nb_params
                     v.use = v.use && __float_as_int(hd.w) != -1;
                     v.inref = true;
                     if (win) {
-                        const int2 W = L.W[__builtin_amdgcn_ubfe(w, 10, 6)];
-                        const int m = W.y >> 31;
-                        const int ok = L.okey[(W.y & 1023) + io];
+                        const int e = (int)__builtin_amdgcn_ubfe(w, 10, 6);
+                        const int ok = L.okey[((L.E[e].x >> 17) & 15) * R + io], kj = (int)(w >> 16);
                         /* key_j + dnshift - key_i < dmaxdist, i and j in task order */
-                        v.inref = ((ok - (int)(w >> 16)) ^ m) - m + W.x > 0;
+                        v.inref = (side ? kj - ok : ok - kj) + L.W[e] > 0;
                         if (!PROJ) v.use = v.use && v.inref;
                     }
                     if (v.use && fabsf(v.r2 - P.rc2f) <= P.band) {
@@ -464,15 +475,19 @@ __device__ __forceinline__ void pair_body(pair_lds<R> &L, const struct nb_params
                     }
                     v.ir = __builtin_amdgcn_rsqf(v.r2);
                     const float r = v.r2 * v.ir;
-                    /* a pair not used reads some interval, or past the
-                       coefficients' end (buffer loads return zeros there) */
                     const unsigned int hw = __float_as_uint(hd.w);
                     const int n = (int)(hw & 511u);
                     int ind = (int)fmaxf(0.0f, hd.x + r * (hd.y + r * hd.z));
                     ind = ind > n ? n : ind;
-                    const int off = (int)(32u * ((hw >> 9) + (unsigned int)ind));
-                    v.a = ld_f4(rs_coef, off);
-                    v.b = ld_f4(rs_coef, off + 16);
+                    const unsigned int off = 32u * ((hw >> 9) + (unsigned int)ind);
+                    if (TABS == 2) {
+                        const float4 *c = (const float4 *)(tab + P.ptab_bytes + (v.use ? off : 0u));
+                        v.a = c[0];
+                        v.b = c[1];
+                    } else {
+                        v.a = ld_f4(rs_coef, v.use ? (int)off : -32);
+                        v.b = ld_f4(rs_coef, v.use ? (int)off + 16 : -16);
+                    }
                 };
                 /* its polynomial, force and sums */
                 auto apply = [&](auto iside, const pair_eval &v) {
