@@ -16,6 +16,7 @@
 #include <time.h>
 
 #include "engine_gpu.h"
+#include "hostpack.h"
 #include "mdcore.h"
 
 int engine_err = engine_err_ok;
@@ -326,7 +327,7 @@ int engine_advance(struct engine *e) {
     /* the energy sum in cell order */
     for (cid = 0; cid < s->nr_real; cid++) epot += s->cells[s->cid_real[cid]].epot;
     /* the kick-drift of every particle, each its own: in parallel */
-#pragma omp parallel for schedule(static) private(pid, k, w)
+#pragma omp parallel for num_threads(space_threads(s->nr_parts)) schedule(static) private(pid, k, w)
     for (cid = 0; cid < s->nr_real; cid++) {
         struct cell *c = &s->cells[s->cid_real[cid]];
         for (pid = 0; pid < c->count; pid++) {
@@ -451,7 +452,7 @@ int engine_finalize(struct engine *e) {
 int engine_getforces(struct engine *e, double *f, int N) {
     int id, k;
     if (e == NULL || f == NULL) return eerror_(engine_err_null);
-#pragma omp parallel for schedule(static) private(k) if (N >= ENGINE_GET_PAR)
+#pragma omp parallel for num_threads(space_threads(N)) schedule(static) private(k) if (N >= ENGINE_GET_PAR)
     for (id = 0; id < N; id++) {
         const struct part *p = (id < e->s.size_parts) ? e->s.partlist[id] : NULL;
         for (k = 0; k < 3; k++) f[3 * (size_t)id + k] = p ? p->f[k] : 0.0;
@@ -462,7 +463,7 @@ int engine_getforces(struct engine *e, double *f, int N) {
 int engine_getpositions(struct engine *e, double *x, int N) {
     int id, k, bad = 0;
     if (e == NULL || x == NULL) return eerror_(engine_err_null);
-#pragma omp parallel for schedule(static) private(k) reduction(| : bad) if (N >= ENGINE_GET_PAR)
+#pragma omp parallel for num_threads(space_threads(N)) schedule(static) private(k) reduction(| : bad) if (N >= ENGINE_GET_PAR)
     for (id = 0; id < N; id++) {
         const struct part *p = (id < e->s.size_parts) ? e->s.partlist[id] : NULL;
         if (p == NULL) {
@@ -481,7 +482,7 @@ int engine_getpositions(struct engine *e, double *x, int N) {
 int engine_getvelocities(struct engine *e, double *v, int N) {
     int id, k, bad = 0;
     if (e == NULL || v == NULL) return eerror_(engine_err_null);
-#pragma omp parallel for schedule(static) private(k) reduction(| : bad) if (N >= ENGINE_GET_PAR)
+#pragma omp parallel for num_threads(space_threads(N)) schedule(static) private(k) reduction(| : bad) if (N >= ENGINE_GET_PAR)
     for (id = 0; id < N; id++) {
         const struct part *p = (id < e->s.size_parts) ? e->s.partlist[id] : NULL;
         if (p == NULL) {

@@ -1,7 +1,24 @@
 /* Host packing between cells and the device's cell-ordered arrays; see
    hostpack.h.  Each loop runs over cells in parallel; every cell writes its
    own slot range, so the results do not depend on the thread count. */
+#include <omp.h>
+
 #include "hostpack.h"
+
+/* A loop takes a thread per SPACE_PER_THREAD particles.  The threads of a team
+   wait for the next loop actively; a team of all 16 cores for every loop used
+   up the process's CPU share, and then the whole process stood still for 20
+   to 50 ms.  32,000 particles, 25 surrogate steps a call, mean and longest of
+   200 calls: 13.5 to 15.1 ms and 64 with 16 threads always, 11.7 and 13.7 with
+   one per 8192, 11.6 and 13.2 per 4096, 11.8 and 14.6 per 16384, 11.9 and 15.2
+   per 32768.  Passes of 64,000 particles 0.77, 0.76, 0.76, 0.78, 0.90 ms, of
+   100,000 0.95, 0.94, 0.96, 0.97, 1.13. */
+#define SPACE_PER_THREAD 8192
+
+int space_threads(int n) {
+    const int m = omp_get_max_threads(), t = 1 + n / SPACE_PER_THREAD;
+    return t < m ? t : m;
+}
 
 int space_pack(const struct space *s, int max_type, int *count, int *offset, int *cnt_off, double *x, int *type,
                int *id, int *maxc, int *maxid) {
@@ -17,7 +34,7 @@ int space_pack(const struct space *s, int max_type, int *count, int *offset, int
         n += c;
     }
     offset[nc] = n;
-#pragma omp parallel for schedule(static) reduction(max : mid) reduction(| : bad)
+#pragma omp parallel for num_threads(space_threads(s->nr_parts)) schedule(static) reduction(max : mid) reduction(| : bad)
     for (int cid = 0; cid < nc; cid++) {
         const struct cell *c = &s->cells[cid];
         for (int k = 0; k < c->count; k++) {
@@ -38,7 +55,7 @@ int space_pack(const struct space *s, int max_type, int *count, int *offset, int
 }
 
 void space_pack_v(const struct space *s, const int *offset, double *v) {
-#pragma omp parallel for schedule(static)
+#pragma omp parallel for num_threads(space_threads(s->nr_parts)) schedule(static)
     for (int cid = 0; cid < s->nr_cells; cid++) {
         const struct cell *c = &s->cells[cid];
         for (int k = 0; k < c->count; k++)
@@ -48,7 +65,7 @@ void space_pack_v(const struct space *s, const int *offset, double *v) {
 
 int space_add_forces(struct space *s, const int *ioi, int n, const float *fhi, const float *flo) {
     int bad = 0;
-#pragma omp parallel for schedule(static) reduction(| : bad)
+#pragma omp parallel for num_threads(space_threads(s->nr_parts)) schedule(static) reduction(| : bad)
     for (int cid = 0; cid < s->nr_cells; cid++) {
         struct cell *c = &s->cells[cid];
         for (int k = 0; k < c->count; k++) {
@@ -65,7 +82,7 @@ int space_add_forces(struct space *s, const int *ioi, int n, const float *fhi, c
 }
 
 void space_add_forces_slots(struct space *s, const int *offset, const float *fhi, const float *flo) {
-#pragma omp parallel for schedule(static)
+#pragma omp parallel for num_threads(space_threads(s->nr_parts)) schedule(static)
     for (int cid = 0; cid < s->nr_cells; cid++) {
         struct cell *c = &s->cells[cid];
         for (int k = 0; k < c->count; k++) {

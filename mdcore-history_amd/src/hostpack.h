@@ -10,6 +10,9 @@
 extern "C" {
 #endif
 
+/* Threads of a host loop over n particles. */
+int space_threads(int n);
+
 /* Cell-ordered slots: count[c], offset[c] (offset[nr_cells] = total),
    cnt_off[2c..2c+1] = (count, offset); x (3 per slot), type, id.  *maxc =
    largest count, *maxid = largest id.  Returns -1 if a type is outside

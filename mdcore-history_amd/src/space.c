@@ -22,6 +22,7 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include "hostpack.h"
 #include "mdcore.h"
 
 int space_err = space_err_ok;
@@ -362,7 +363,7 @@ int space_prepare(struct space *s) {
     s->virial = 0.0;
     s->nr_pairs = 0;
     s->nr_excl_evaluated = 0;
-#pragma omp parallel for schedule(static) private(pid, k)
+#pragma omp parallel for num_threads(space_threads(s->nr_parts)) schedule(static) private(pid, k)
     for (cid = 0; cid < s->nr_cells; cid++) {
         struct cell *c = &s->cells[cid];
         c->epot = 0.0;
@@ -384,7 +385,7 @@ int space_shuffle_local(struct space *s) {
     struct part *p;
     unsigned char *leaves = (unsigned char *)malloc(s->nr_real > 0 ? (size_t)s->nr_real : 1);
     if (leaves == NULL) return serror_(space_err_malloc);
-#pragma omp parallel for schedule(static) private(pid, k)
+#pragma omp parallel for num_threads(space_threads(s->nr_parts)) schedule(static) private(pid, k)
     for (cid = 0; cid < s->nr_real; cid++) {
         const struct cell *cc = &s->cells[s->cid_real[cid]];
         unsigned char out = 0;
@@ -421,7 +422,7 @@ int space_shuffle_local(struct space *s) {
     free(leaves);
     /* each cell appends its own newcomers and rewrites its own particles'
        partlist entries */
-#pragma omp parallel for schedule(static) reduction(| : bad)
+#pragma omp parallel for num_threads(space_threads(s->nr_parts)) schedule(static) reduction(| : bad)
     for (cid = 0; cid < s->nr_marked; cid++)
         bad |= cell_welcome(&s->cells[s->cid_marked[cid]], s->partlist) < 0;
     if (bad) return serror_(space_err_cell);
@@ -466,7 +467,7 @@ int space_setcells(struct space *s, const int *count, const double *x, const dou
     }
     meta = (struct meta *)s->setcells_scratch;
     start = (int *)(meta + (n > 0 ? n : 1));
-#pragma omp parallel for schedule(static) reduction(| : bad)
+#pragma omp parallel for num_threads(space_threads(s->nr_parts)) schedule(static) reduction(| : bad)
     for (a = 0; a < n; a++) {
         if (id[a] < 0 || id[a] >= s->size_parts || s->partlist[id[a]] == NULL) {
             bad = 1;
@@ -484,7 +485,7 @@ int space_setcells(struct space *s, const int *count, const double *x, const dou
         a += count[cid];
         if (count[cid] > c->size && cell_grow(c, count[cid]) < 0) return serror_(space_err_malloc);
     }
-#pragma omp parallel for schedule(static)
+#pragma omp parallel for num_threads(space_threads(s->nr_parts)) schedule(static)
     for (cid = 0; cid < s->nr_cells; cid++) {
         struct cell *c = &s->cells[cid];
         for (int k = 0; k < count[cid]; k++) {
