@@ -53,8 +53,8 @@ MI355X_CUS = 256
 DT_PS = 0.002               # 2 fs time step for ns/day
 MLP_TRAIN_STEPS = 40000     # surrogate training steps on the mixture (16,384 samples each)
 METRIC = "pair-interactions/s & ns/day at 1M atoms; MLP vs table at fixed force RMSE"
-TRAFFIC_FILE = ROOT / "profiles" / "k_nonbond_mixture_1m_traffic.json"
-COUNTERS_FILE = ROOT / "profiles" / "k_nonbond_mixture_1m_counters.json"
+TRAFFIC_FILE = ROOT / "profiles" / "k_pair_mixture_1m_traffic.json"
+COUNTERS_FILE = ROOT / "profiles" / "k_pair_mixture_1m_counters.json"
 
 
 _T0 = time.perf_counter()

@@ -121,7 +121,8 @@ int engine_gpu_steps(struct engine *e, int nsteps, double *epot, double *ekin);
    engine_gpu_half_mean atoms or more on average and are fewer than the
    device's compute units (or engine_flag_unpaired is set).  Otherwise the
    full shell is taken: the half shell's opposite forces, LDS atomics, cost
-   more than the evaluations they save.
+   more than the evaluations they save.  (With few cells engine_flag_fullshell
+   is faster too, with the energy's sums in another order.)
    The surrogate pass (engine_flag_mlp) takes the half shell unless
    engine_flag_fullshell is set: its network evaluation dominates a visit. */
 #define engine_flag_fullshell 262144

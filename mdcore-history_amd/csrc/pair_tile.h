@@ -44,7 +44,7 @@
  * key_j + dnshift - key_i <= dscale (x_j + shift - x_i).n + 1 <= dscale rc + 1
  * < dmaxdist for every pair within the cutoff.
  *
- * What bounds it: VALU issue (85 % busy on 20 types), 71 instructions per hit
+ * What bounds it: VALU issue (84 % busy on 20 types), 71 instructions per hit
  * and lane on the i side at half the lanes busy (an atom's hits per chunk
  * differ), 60 on the j side at 97 %; with 20 types the coefficients come next,
  * 384 KB of tables read at random through the 32 KB L1.  The L1 serves about a
