@@ -258,6 +258,10 @@ __global__ __launch_bounds__(256) void k_clear_ids(int nids, int *__restrict__ i
     if (k < nids) index_of_id[k] = -1;
 }
 
+__global__ __launch_bounds__(64) void k_clear_queue(int *__restrict__ queue) {
+    if (threadIdx.x < MD_NQUEUE) queue[threadIdx.x] = 0;
+}
+
 /* ------------------------------------------------------------ k_sort */
 
 #define MD_SORT_STACK 16
@@ -2452,7 +2456,7 @@ extern "C" int engine_gpu_load(struct engine *e) {
     HIPCHECK(hipMalloc(&g->d_red_cnt, sizeof(unsigned long long) * 3 * MD_RED_BLOCKS));
     HIPCHECK(hipMalloc(&g->d_tot_cnt, sizeof(unsigned long long) * 4));
     HIPCHECK(hipMalloc(&g->d_queue, sizeof(int) * MD_NQUEUE));
-    HIPCHECK(hipMemset(g->d_queue, 0, sizeof(int) * MD_NQUEUE)); /* each pass leaves it zero */
+    g->queue_used = 1;
     HIPCHECK(hipHostMalloc((void **)&g->h_count, sizeof(int) * s->nr_cells, hipHostMallocDefault));
     HIPCHECK(hipMalloc(&g->d_cell_maxdx, sizeof(double) * s->nr_cells));
     HIPCHECK(hipHostMalloc((void **)&g->h_cell_maxdx, sizeof(double) * s->nr_cells, hipHostMallocDefault));
@@ -2672,6 +2676,9 @@ int gpu_launch(struct gpu_state *g, int timed, int mlp, int sort, int packed) {
                            g->d_kminmax, g->d_sortlist, g->d_keyof, g->d_ptab, (const float4 *)g->d_coeffs,
                            g->d_excl_off, g->d_excl_list, g->d_index_of_id, g->d_cell_of, O);
     } else {
+        /* new, or left used up by a pass that ended in an error before its totals */
+        if (g->queue_used) hipLaunchKernelGGL(k_clear_queue, dim3(1), dim3(64), 0, g->stream, g->d_queue);
+        g->queue_used = 1;
         /* no more waves than work items: the dispatcher then spreads them
            over all compute units */
         const dim3 grid(g->grid_nb[kern] < nitems ? g->grid_nb[kern] : nitems);
@@ -2706,6 +2713,7 @@ int gpu_launch(struct gpu_state *g, int timed, int mlp, int sort, int packed) {
     }
     if (timed) HIPCHECK(hipEventRecord(g->ev[3], g->stream));
     HIPCHECK(hipGetLastError());
+    g->queue_used = 0;
     return engine_err_ok;
 }
 

@@ -111,6 +111,7 @@ struct gpu_state {
     double *d_red_acc; /* per-block partial sums of the totals */
     unsigned long long *d_red_cnt;
     int *d_queue;
+    int queue_used; /* not known to be zero, as the totals of a pass leave it */
     int *d_order; /* owner cells in blocked work order */
     /* pseudo-Verlet: per-cell maxdx on the device; whether the sort lists
        are those of the last sort of the current layout, and its counts */
