@@ -72,6 +72,8 @@
 #define PT_LS 18     /* i side: half words of a lane's list; 9 words, so that lanes differ in bank */
 #define PT_WAVES 4   /* items per block: they share the LDS copy of the tables */
 #define PT_TAB 8192  /* bytes of LDS for table headers and coefficients */
+#define PT_FAR 1.8e19f /* coordinates of a slot without an atom: its r^2 is infinite, whatever the
+                          length unit, so it passes neither the filter nor the cutoff */
 
 typedef float pt_f4 __attribute__((ext_vector_type(4)));
 
@@ -212,13 +214,12 @@ __device__ __forceinline__ void pair_body(pair_lds<R> &L, const char *tab, const
         if (ilane)
             for (int b = part; b < 64; b += NP) recs |= 1ull << b;
 
-        /* Owner atoms: records, keys.  Lanes past nsub place far-away atoms
-           in the last tile's empty columns. */
+        /* Owner atoms: records, keys.  The last tile's empty columns hold any
+           atoms: nothing reads their bits. */
         wave_lds_sync();
         if (lane < R) {
             const bool in = lane < nsub;
-            L.own[lane] = make_float4(in ? xo.x : 1.0e4f, in ? xo.y : 1.0e4f, in ? xo.z : 1.0e4f,
-                                      __int_as_float(16 * mt * to));
+            L.own[lane] = make_float4(xo.x, xo.y, xo.z, __int_as_float(16 * mt * to));
             if (P.window && in)
                 for (int sid = 0; sid < 13; sid++) L.okey[sid * R + lane] = keyof[(size_t)sid * P.nparts + a];
         }
@@ -352,7 +353,7 @@ __device__ __forceinline__ void pair_body(pair_lds<R> &L, const char *tab, const
 #pragma unroll
                     for (int s = 0; s < NB; s++) {
                         const int t = 64 * s + lane;
-                        float4 p = make_float4(1.0e4f, 1.0e4f, 1.0e4f, 0.f);
+                        float4 p = make_float4(PT_FAR, PT_FAR, PT_FAR, 0.f);
                         if (in[s]) {
                             p.x = x[s].x + sh[s].x;
                             p.y = x[s].y + sh[s].y;

@@ -92,3 +92,11 @@ def check_forces(s, flags, proj, unit=1.0):
 @pytest.mark.parametrize("r", [32, 64])
 def test_every_pair_on_both_sides(r, ntypes, flags, proj):
     check_forces(crowd(r, ntypes, 100 * r + ntypes), flags, proj)
+
+
+# cells and cutoff of 1e4 length units, and the null type 0 with potentials
+# and atoms of its own: slots without an atom must not count as atoms
+@pytest.mark.parametrize("proj", [False, True])
+@pytest.mark.parametrize("r", [32, 64])
+def test_length_unit_and_type_zero(r, proj):
+    check_forces(crowd(r, 2, 7 + r, unit=1e4, first=0), 0, proj, unit=1e4)
