@@ -2246,10 +2246,9 @@ extern "C" int engine_gpu_load(struct engine *e) {
     }
 
     /* Half-shell lists: the self task and each pair task once, at the task's
-       i cell, in the order of the full-shell list; for each cell the i cells
-       that visit it as the task's j cell, in task order, each at slot
-       1 + its position (slot 0 is the self task), which the entry carries in
-       its bits 9 and up. */
+       i cell, and for each cell the i cells that visit it as the task's j
+       cell, all in task order; of the latter each has slot 1 + its position
+       (slot 0 is the self task), which the entry carries in its bits 9 and up. */
     {
         const int nc = s->nr_cells;
         int *hcnt = (int *)calloc(nc + 1, sizeof(int)), *icnt = (int *)calloc(nc + 1, sizeof(int));
@@ -2286,25 +2285,22 @@ extern "C" int engine_gpu_load(struct engine *e) {
             icell = (int *)malloc(sizeof(int) * (itot > 0 ? itot : 1));
             if (nbr == NULL || nbs == NULL || icell == NULL) bad = 1;
         }
-        /* entries without a window test first (win 0), then the others */
-        for (int win = 0; !bad && win < 2; win++)
-            for (k = 0; k < s->nr_tasks; k++) {
-                const struct task *t = &s->tasks[k];
-                if (t->type == task_type_self && win == 0) {
-                    const int en = hfill[t->i]++;
-                    nbs[en] = make_float4(0.f, 0.f, 0.f, 0.f);
-                    nbr[en] = make_int4(t->i, 1 << 5, 0, 0);
-                } else if (t->type == task_type_pair) {
-                    int dr, dp;
-                    task_dnshift(s, t->i, t->j, t->flags, g->P.dscale, &dr, &dp);
-                    if (task_window(g, s, dr, dp) != win) continue;
-                    const int en = hfill[t->i]++;
-                    const int slot = 1 + ifill[t->j] - ioff[t->j];
-                    nbs[en] = cell_shift32(s, t->i, t->j);
-                    nbr[en] = make_int4(t->j, t->flags | (win << 8) | (slot << 9), dr, dp);
-                    icell[ifill[t->j]++] = t->i;
-                }
+        for (k = 0; !bad && k < s->nr_tasks; k++) {
+            const struct task *t = &s->tasks[k];
+            if (t->type == task_type_self) {
+                const int en = hfill[t->i]++;
+                nbs[en] = make_float4(0.f, 0.f, 0.f, 0.f);
+                nbr[en] = make_int4(t->i, 1 << 5, 0, 0);
+            } else if (t->type == task_type_pair) {
+                int dr, dp;
+                const int en = hfill[t->i]++;
+                const int slot = 1 + ifill[t->j] - ioff[t->j];
+                task_dnshift(s, t->i, t->j, t->flags, g->P.dscale, &dr, &dp);
+                nbs[en] = cell_shift32(s, t->i, t->j);
+                nbr[en] = make_int4(t->j, t->flags | (slot << 9), dr, dp);
+                icell[ifill[t->j]++] = t->i;
             }
+        }
         if (!bad) {
             if (hipMalloc(&g->d_nbr_h, sizeof(int4) * (htot > 0 ? htot : 1)) != hipSuccess ||
                 hipMalloc(&g->d_nbs_h, sizeof(float4) * (htot > 0 ? htot : 1)) != hipSuccess ||

@@ -54,8 +54,9 @@ struct nb_params {
 };
 
 /* Neighbour-list entry of an owner cell: x = other cell, y = sid | orient<<4
-   | self<<5 | window<<8 (orient 0: owner is the task's i cell; window: see
-   pair_tile.h; half shell: jpart slot<<9, else distance class<<16), z = dnshift with the reference window |shift|, w = dnshift with the projected shift.n.
+   | self<<5 (orient 0: owner is the task's i cell) | full shell: window<<8 (see
+   pair_tile.h) | distance class<<16; half shell: jpart slot<<9; z = dnshift with
+   the reference window |shift|, w = dnshift with the projected shift.n.
    Type-pair table header ptab[ti*mt+tj] = (alpha0, alpha1, alpha2,
    bits(n | chunk0 << 9)) or w = bits(-1) when the pair has no potential. */
 
