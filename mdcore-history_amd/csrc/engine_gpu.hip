@@ -2482,6 +2482,9 @@ int gpu_upload(struct engine *e) {
     if (maxc > g->maxcell)
         return gerror_(engine_err_maxparts, "more particles in a cell than the packed record holds (1024 for up to "
                                             "64 types, 256 for up to 256, 64 for up to 1024)");
+    /* the copy of an upload whose call ended in an error before its end */
+    if (g->staging) HIPCHECK(hipStreamSynchronize(g->stream));
+    g->staging = 0;
     if (gpu_alloc_parts(g, n > 0 ? n : 1) < 0) return engine_err_gpu;
     /* the id clearing runs while the host packs */
     if (gpu_clear_ids(g) < 0) return engine_err_gpu;
@@ -2515,6 +2518,7 @@ int gpu_upload(struct engine *e) {
     g->P.nparts = n;
     g->P.nids = g->nids;
     g->P.maxn = maxc > 0 ? maxc : 1;
+    g->staging = 1;
     HIPCHECK(hipMemcpyAsync(g->d_stage, g->h_stage, GPU_STAGE_BYTES(n, s->nr_cells), hipMemcpyHostToDevice, g->stream));
     {
         const double *x = (const double *)g->d_stage;
@@ -2724,6 +2728,7 @@ extern "C" int engine_gpu_sync(struct engine *e, unsigned int what) {
     if (what & engine_gpu_sync_parts_up) {
         if (gpu_upload(e) < 0) return engine_err_gpu;
         HIPCHECK(hipStreamSynchronize(g->stream));
+        g->staging = 0;
     }
     if (what & engine_gpu_sync_sort_down) {
         unsigned int *tmp = (unsigned int *)malloc(sizeof(unsigned int) * 13 * (size_t)(g->nparts > 0 ? g->nparts : 1));
@@ -2808,6 +2813,7 @@ extern "C" int engine_nonbond_gpu(struct engine *e) {
     HIPCHECK(hipMemcpyAsync(g->h_fhi, g->d_fhi, sizeof(float4) * 2 * g->nparts, hipMemcpyDeviceToHost, g->stream));
     if (sort) gpu_sorted(e, g); /* meanwhile */
     HIPCHECK(hipStreamSynchronize(g->stream));
+    g->staging = 0;
     if (*(const volatile int *)g->h_flag) return gerror_(engine_err_range, "sort stack overflow");
     {
         float ms = 0.0f;

@@ -122,6 +122,7 @@ struct gpu_state {
        offset) of the uploaded particles, one after the other) and its copy on
        the device; flo follows fhi in the same block */
     char *h_stage, *d_stage;
+    int staging; /* a copy from h_stage has not been waited for */
     int *h_flag; /* pinned: set by a sort that overflows */
     double *h_x;
     int *h_type, *h_id, *h_count, *h_offset;

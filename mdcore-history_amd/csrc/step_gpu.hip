@@ -1290,7 +1290,7 @@ extern "C" int engine_gpu_steps(struct engine *e, int nsteps, double *epot, doub
         rc = gerror_(engine_err_gpu, "step failed");
     if (rc == engine_err_ok && *(const volatile int *)g->h_flag) rc = gerror_(engine_err_range, "sort stack overflow");
     if (rc == engine_err_ok) rc = step_download(e, g, &b, nsteps, epot, ekin, verlet, smaxdx);
-    (void)hipStreamSynchronize(g->stream);
+    if (hipStreamSynchronize(g->stream) == hipSuccess) g->staging = 0;
     step_free_rigid(&b);
     step_put(g, &b);
     /* without pseudo-Verlet the last sort lists belong to the layout before
