@@ -2,6 +2,7 @@
    hostpack.h.  Each loop runs over cells in parallel; every cell writes its
    own slot range, so the results do not depend on the thread count. */
 #include <omp.h>
+#include <pthread.h>
 
 #include "hostpack.h"
 
@@ -15,9 +16,20 @@
    100,000 0.95, 0.94, 0.96, 0.97, 1.13. */
 #define SPACE_PER_THREAD 8192
 
+/* A child forked after a loop of several threads has none of them, and
+   libgomp would wait for them: its loops take one. */
+static volatile int teams, alone;
+
+static void forked(void) { alone |= teams; }
+
+__attribute__((constructor)) static void watch_forks(void) { (void)pthread_atfork(NULL, NULL, forked); }
+
 int space_threads(int n) {
-    const int m = omp_get_max_threads(), t = 1 + n / SPACE_PER_THREAD;
-    return t < m ? t : m;
+    const int m = alone ? 1 : omp_get_max_threads();
+    int t = 1 + n / SPACE_PER_THREAD;
+    t = t < m ? t : m;
+    if (t > 1 && !teams) teams = 1;
+    return t;
 }
 
 int space_pack(const struct space *s, int max_type, int *count, int *offset, int *cnt_off, double *x, int *type,
