@@ -765,15 +765,19 @@ __device__ __forceinline__ void pair_body(pair_lds<R> &L, const char *tab, const
         }
 
         /* the partitions' sums, in order, into the atoms' */
+        double px = 0.0, py = 0.0, pz = 0.0;
         for (int p = 1; p * nsub < 64; p++) {
             const int l = lane + p * nsub;
             const double ax = __shfl(hx, l & 63), ay = __shfl(hy, l & 63), az = __shfl(hz, l & 63);
             if (lane < nsub && l < 64) {
-                hx += ax;
-                hy += ay;
-                hz += az;
+                px += ax;
+                py += ay;
+                pz += az;
             }
         }
+        hx += px;
+        hy += py;
+        hz += pz;
 
         /* Excluded pairs: subtract what the pair pass added
            (exclusion.c:139-208), same FP32 arithmetic. */
