@@ -146,11 +146,11 @@ __device__ __forceinline__ float4 ld_f4(__amdgpu_buffer_rsrc_t r, int byte_off) 
     return out;
 }
 
-/* pot_eval32 for two pairs at once, without branches: both coefficient
+/* pot_eval32r for two pairs at once, without branches: both coefficient
    rows are requested before either polynomial is evaluated, so the two
    table lookups overlap.  A pair with use_* false (no hit, or no table for
    its types) reads interval 0 of the first table instead and returns
-   e = f = 0. */
+   e = f = 0; the arithmetic of a used pair is that of pot_eval32r. */
 __device__ __forceinline__ void pot_eval32r2(const float4 ha, const float4 hb, bool use_a, bool use_b,
                                              __amdgpu_buffer_rsrc_t rc, float r2a, float r2b, float &ea,
                                              float &fa, float &eb, float &fb) {
@@ -2556,6 +2556,7 @@ int gpu_launch(struct gpu_state *g, int timed, int mlp, int sort, int packed) {
        them (measured equal to 4 at 64 cells per CU, ahead above) */
     const int wide = !mlp && half && g->ncells >= 64 * g->ncu;
     struct nb_params P = g->P;
+    P.walk_cap = g->ncells >= 64 * g->ncu ? MD_HCAP_WIDE : MD_HCAP;
     const int nsplit = P.nsplit = pair ? g->nsplit_t : g->nsplit;
     int nb;
     size_t lds = 0;

@@ -51,6 +51,7 @@ struct nb_params {
     const int *order; /* owner cell of each owner position in the work order */
     int window; /* some entries need the reference's window test (pair_tile.h) */
     float filt; /* k_pair's filter threshold on r^2 */
+    int walk_cap; /* k_pair, projected window: see pair_tile.h */
 };
 
 /* Neighbour-list entry of an owner cell: x = other cell, y = sid | orient<<4

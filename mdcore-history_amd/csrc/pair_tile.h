@@ -130,12 +130,19 @@ __device__ __forceinline__ unsigned int wave_incl_scan_u32(unsigned int v) {
 }
 
 /* Table lookup of one pair in two steps, so that the coefficients' load can
-   be in flight while another pair is worked on: pot_eval32's arithmetic. */
+   be in flight while another pair is worked on: pot_eval32r's arithmetic. */
 struct pair_eval {
     float dx, dy, dz, ir, r2;    /* the pair */
     float4 a, b;                 /* its interval's coefficients */
-    bool use, inref;             /* evaluated; inside the reference window */
+    bool use, inref, odd;        /* evaluated; inside the reference window; see `parity` */
 };
+
+/* r - c with r = r2 ir rounded first. */
+__device__ __forceinline__ float pt_offset(float r2, float ir, float c) {
+#pragma clang fp contract(off)
+    const float r = r2 * ir;
+    return r - c;
+}
 
 /* TABS: 1, 2: the table headers (and 2: the coefficients) are in LDS at tab.
    PROJ: the projected window (every pair within the cutoff); the pass also
@@ -294,6 +301,13 @@ __device__ __forceinline__ void pair_body(pair_lds<R> &L, const char *tab, const
                had a hit in the entry of the last piece */
             float le = 0.f, lv = 0.f;
             bool seen = false;
+            /* PROJ: the walk along the sorted lists that these sums are held
+               to, bit for bit, evaluated a lane's hits of walk_cap records two
+               at a time and rounded r in the second before subtracting the
+               interval's centre (in the first of the two it did not) */
+            bool parity = false;
+            int rnd = 0;
+            const float rnd_inv = __builtin_amdgcn_rcpf((float)(P.walk_cap * NP)) * 1.0001f;
             /* chunks of equal size, a multiple of 4 slots */
             const int nck = (total + PT_TC - 1) / PT_TC;
             const int tck = ((total + nck - 1) / nck + 3) & ~3;
@@ -415,6 +429,7 @@ __device__ __forceinline__ void pair_body(pair_lds<R> &L, const char *tab, const
                 double fx = 0.0, fy = 0.0, fz = 0.0; /* j side: of the run */
                 unsigned int cur = 0u; /* hits left in the lane's word */
                 int tb = 0;            /* 16 x its first slot */
+                int tt = 0;            /* i side: its first record in the entry */
                 /* the pair of hit s of `mine`, owner atom (xi, io):
                    geometry, window and cutoff tests, its coefficients
                    requested */
@@ -433,6 +448,14 @@ __device__ __forceinline__ void pair_body(pair_lds<R> &L, const char *tab, const
                     v.dz = xi.z - pj.z;
                     v.r2 = v.dx * v.dx + v.dy * v.dy + v.dz * v.dz;
                     v.use = have && v.r2 <= rc2hi;
+                    v.odd = false;
+                    if (PROJ && !side) {
+                        const int b = have ? (int)((float)(tt + bit) * rnd_inv) : rnd;
+                        if (b != rnd) parity = false;
+                        rnd = b;
+                        v.odd = parity;
+                        parity = parity != v.use;
+                    }
                     v.use = v.use && __float_as_int(hd.w) != -1;
                     v.inref = true;
                     if (win) {
@@ -481,7 +504,10 @@ __device__ __forceinline__ void pair_body(pair_lds<R> &L, const char *tab, const
                 /* its polynomial, force and sums */
                 auto apply = [&](auto iside, const pair_eval &v) {
                     if (v.use) {
-                        const float x = fmaf(v.r2, v.ir, -v.a.x) * v.a.y;
+                        float x = fmaf(v.r2, v.ir, -v.a.x);
+                        if constexpr (PROJ && decltype(iside)::value == 1)
+                            if (v.odd) x = pt_offset(v.r2, v.ir, v.a.x);
+                        x *= v.a.y;
                         float ee = v.a.z * x + v.a.w;
                         float eff = v.a.z;
                         eff = eff * x + ee;
@@ -573,7 +599,13 @@ __device__ __forceinline__ void pair_body(pair_lds<R> &L, const char *tab, const
                             pmask &= pmask - 1u;
                             cur = lst[q];
                             tb = L.slot[q0 + q];
-                            return (first >> q) & 1u;
+                            const bool begins = (first >> q) & 1u;
+                            if (PROJ) {
+                                const unsigned int pd = L.piece[q0 + q];
+                                tt = (int)((pd >> 13) & 0x7ffu);
+                                if (begins) parity = false;
+                            }
+                            return begins;
                         };
                         auto flush = [&](bool yes) {
                             if (yes) {

@@ -72,24 +72,3 @@ def test_large_forces_that_cancel(nw, flags, proj):
         assert np.all(err <= 3e-6 * weak + 100 * 2.0 ** -28), (err / weak).max()
     finally:
         e.close()
-
-
-# where both windows admit the same pairs their energies are the same bits: a
-# pair's arithmetic does not depend on its place in the walk
-@pytest.mark.parametrize("flags", [0, md.engine_flag_nosplit])
-@pytest.mark.parametrize("nw", [4, 30])
-def test_energies_of_both_windows(nw, flags):
-    s = crystal(nw)
-    o = po.from_system(s)
-    assert o.nonbond(po.OR_WINDOW_REF)["pairs"] == o.nonbond(po.OR_WINDOW_PROJ)["pairs"]
-    out = []
-    for proj in (0, md.engine_flag_projwindow):
-        e = systems.build_engine(s, md.engine_flag_gpu | md.engine_flag_fullshell | flags | proj)
-        try:
-            e.shuffle()
-            e.nonbond()
-            en = e.energies()
-            out.append((en["epot_nonbond"], en["virial"], en["pairs"]))
-        finally:
-            e.close()
-    assert out[0] == out[1]
