@@ -146,11 +146,11 @@ __device__ __forceinline__ float4 ld_f4(__amdgpu_buffer_rsrc_t r, int byte_off) 
     return out;
 }
 
-/* pot_eval32r for two pairs at once, without branches: both coefficient
+/* pot_eval32 for two pairs at once, without branches: both coefficient
    rows are requested before either polynomial is evaluated, so the two
    table lookups overlap.  A pair with use_* false (no hit, or no table for
    its types) reads interval 0 of the first table instead and returns
-   e = f = 0; the arithmetic of a used pair is that of pot_eval32r. */
+   e = f = 0. */
 __device__ __forceinline__ void pot_eval32r2(const float4 ha, const float4 hb, bool use_a, bool use_b,
                                              __amdgpu_buffer_rsrc_t rc, float r2a, float r2b, float &ea,
                                              float &fa, float &eb, float &fb) {
@@ -941,6 +941,7 @@ __device__ __forceinline__ void mlp_dense_eval(const struct mlp_net &N, const fl
 #define MD_PAIR_ITEMS_PER_CU 12  /* k_pair: work items per CU that owners are split up to */
 #define MD_PAIR_SPLIT_MAX 32     /* k_pair: at most this many groups (of two entries at least) */
 #define MD_PAIR_R64_MEAN 32      /* atoms per cell above which k_pair takes 64 owner atoms at a time */
+#define MD_WALK_CELLS 16384 /* k_pair, projected window: cells from which walk_cap is 28 (pair_tile.h) */
 #define MD_HCAP 32     /* table mode: hits buffered per lane before they are evaluated */
 #define MD_HCAP_WIDE 28 /* the same in the 5-wave build: its LDS then allows 20 waves per CU */
 #define MD_HCAP_MLP 8  /* MLP mode: hits per lane per compaction round */
@@ -2556,7 +2557,7 @@ int gpu_launch(struct gpu_state *g, int timed, int mlp, int sort, int packed) {
        them (measured equal to 4 at 64 cells per CU, ahead above) */
     const int wide = !mlp && half && g->ncells >= 64 * g->ncu;
     struct nb_params P = g->P;
-    P.walk_cap = g->ncells >= 64 * g->ncu ? MD_HCAP_WIDE : MD_HCAP;
+    P.walk_cap = g->ncells >= MD_WALK_CELLS ? 28 : 32;
     const int nsplit = P.nsplit = pair ? g->nsplit_t : g->nsplit;
     int nb;
     size_t lds = 0;

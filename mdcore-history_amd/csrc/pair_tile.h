@@ -130,14 +130,14 @@ __device__ __forceinline__ unsigned int wave_incl_scan_u32(unsigned int v) {
 }
 
 /* Table lookup of one pair in two steps, so that the coefficients' load can
-   be in flight while another pair is worked on: pot_eval32r's arithmetic. */
+   be in flight while another pair is worked on: pot_eval32's arithmetic. */
 struct pair_eval {
     float dx, dy, dz, ir, r2;    /* the pair */
     float4 a, b;                 /* its interval's coefficients */
     bool use, inref, odd;        /* evaluated; inside the reference window; see `parity` */
 };
 
-/* r - c with r = r2 ir rounded first. */
+/* r - c with r = r2 ir rounded first (every other hit, see `parity`). */
 __device__ __forceinline__ float pt_offset(float r2, float ir, float c) {
 #pragma clang fp contract(off)
     const float r = r2 * ir;
@@ -301,10 +301,13 @@ __device__ __forceinline__ void pair_body(pair_lds<R> &L, const char *tab, const
                had a hit in the entry of the last piece */
             float le = 0.f, lv = 0.f;
             bool seen = false;
-            /* PROJ: the walk along the sorted lists that these sums are held
-               to, bit for bit, evaluated a lane's hits of walk_cap records two
-               at a time and rounded r in the second before subtracting the
-               interval's centre (in the first of the two it did not) */
+            /* PROJ: in every other hit of a lane's walk_cap records r is
+               rounded before the interval's centre is subtracted.  It makes
+               no energy more exact; without it the projected window's totals,
+               FP64 outputs, would differ by 1e-9 to 3e-9 of themselves from
+               those that this library has always given (a kernel that is gone
+               evaluated hits two at a time, walk_cap records a round).  The
+               rule depends on the number of cells alone. */
             bool parity = false;
             int rnd = 0;
             const float rnd_inv = __builtin_amdgcn_rcpf((float)(P.walk_cap * NP)) * 1.0001f;
