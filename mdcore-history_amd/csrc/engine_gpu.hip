@@ -189,7 +189,7 @@ __device__ __forceinline__ void pot_eval32r2(const float4 ha, const float4 hb, b
     fb = use_b ? f2 : 0.f;
 }
 
-/* The pair kernel's workgroup is a single wavefront, and the LDS executes a
+/* A wave of the pair kernels shares its LDS with no other, and the LDS executes a
    wavefront's instructions in order: data written by one lane is visible to
    another lane's later read once this wave's LDS operations have completed.
    This waits for LDS only (lgkmcnt(0)) and keeps the compiler from moving
@@ -2410,7 +2410,8 @@ extern "C" int engine_gpu_load(struct engine *e) {
        per CU: argon 1331 cells 66, 53, 52, 52, 60; mixture 125 cells 120, 114,
        137, 136, 138, 729 cells 170, 122, 114, 134, 132; water 512 cells 408,
        329, 414, 375, 395, 729 cells 706, 497, 575, 546, 574; and unsplit: argon
-       64 cells 82, now 30, mixture 125 cells 618, now 114. */
+       64 cells 82, now 34, mixture 125 cells 618, now 116.  (The sweep with FP32
+       force sums.) */
     g->nsplit_t = 1;
     if (!(e->flags & engine_flag_nosplit)) {
         int cap = g->maxnbr / 2 < MD_PAIR_SPLIT_MAX ? g->maxnbr / 2 : MD_PAIR_SPLIT_MAX;
@@ -2505,8 +2506,8 @@ int gpu_upload(struct engine *e) {
     g->paired = !(e->flags & engine_flag_unpaired);
     /* default shell: the full shell, except for densely filled cells that are
        fewer than the device's CUs, or with engine_flag_unpaired.  There too
-       k_pair is the faster one now (water, 27, 64 and 125 cells of 111 to 168
-       atoms: 228, 279 and 308 us against 275, 361 and 448), but its energy sums
+       k_pair is the faster one now (water, 27, 64 and 125 cells of 111 to 125
+       atoms: 244, 166 and 302 us against 261, 234 and 384), but its energy sums
        run in another order than the half shell's: where pair and exclusion
        energies cancel, the total differs by up to 4e-6 of itself. */
     g->half = (e->flags & engine_flag_halfshell)   ? 1
@@ -2550,7 +2551,7 @@ int gpu_launch(struct gpu_state *g, int timed, int mlp, int sort, int packed) {
        share and registers leave 3 waves per SIMD instead of 4); beyond, the
        cell's neighbours would be staged twice (at 39, 49 and 62 per cell 201,
        226 and 213 us with 32, 135, 157 and 149 with 64; water at 125 per cell
-       434 and 328) */
+       434 and 328; all with FP32 force sums) */
     const int big = (long long)g->nparts > (long long)MD_PAIR_R64_MEAN * g->ncells;
     const int half = mlp ? g->mlp_half : g->half, pair = !mlp && !half;
     /* table mode on the half shell: 5 waves per SIMD where the cells fill
@@ -2664,7 +2665,7 @@ int gpu_launch(struct gpu_state *g, int timed, int mlp, int sort, int packed) {
         /* the tables in LDS as far as PT_TAB bytes hold them: with them 4
            blocks of 4 waves still fit on a CU, and every access kept from the
            L1 counts (argon 864,000 atoms, all in LDS: 622 -> 595 us; 20 types,
-           the headers: 4180 -> 3670 us) */
+           the headers: 4180 -> 3670 us; with FP32 force sums) */
         const int tabs = P.ptab_bytes + P.coef_bytes <= PT_TAB ? 2 : P.ptab_bytes <= PT_TAB ? 1 : 0;
         const size_t plds = PT_WAVES * (big ? sizeof(pair_lds<64>) : sizeof(pair_lds<32>)) +
                             (tabs ? P.ptab_bytes : 0) + (tabs == 2 ? P.coef_bytes : 0);

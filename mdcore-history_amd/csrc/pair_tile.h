@@ -38,9 +38,10 @@
  * chunks, an atom's forces in different cells met in FP32: small ones beside
  * large ones that cancel were lost, and the relative force error of the
  * mixture was 1.381e-6 at 1,048,576 atoms, now 1.373e-6 (FP32 sums over one
- * visited cell: 1.374e-6).  An FP64 FMA issues like an FP32 one; the four
- * conversions per hit cost 5 % (1,048,576 atoms, mixture 3650 -> 3830 us,
- * argon 729 -> 768), nearly all of it on the j side.
+ * visited cell: 1.374e-6).  It adds 1.7 % VALU instructions, four conversions
+ * per hit less the two-sums, and up to 5 % of the time, since the FP64 ones take
+ * more than one issue cycle (1,048,576 atoms, mixture 3650 -> 3830 us, argon
+ * 729 -> 770), nearly all of it on the j side.
  *
  * The set of pairs is the reference's.  Its sorted window
  * (runner_dopair.c:455-478) admits (i, j) exactly when
@@ -51,18 +52,20 @@
  * key_j + dnshift - key_i <= dscale (x_j + shift - x_i).n + 1 <= dscale rc + 1
  * < dmaxdist for every pair within the cutoff.
  *
- * What bounds it: VALU issue (84 % busy on 20 types), 71 instructions per hit
- * and lane on the i side at half the lanes busy (an atom's hits per chunk
- * differ), 60 on the j side at 97 %; with 20 types the coefficients come next,
- * 384 KB of tables read at random through the 32 KB L1.  The L1 serves about a
- * lane a clock, so a lane without a hit asks for nothing (mixture 1,048,576:
+ * What bounds it: the VALU (81 % of its issue cycles filled on 20 types, and the
+ * FP64 instructions take longer), 75 instructions per hit and lane on the i
+ * side at half the lanes busy (an atom's hits per chunk differ), 64 on the j
+ * side at 97 %; with 20 types the coefficients come next, 384 KB of tables read
+ * at random through the 32 KB L1.  The L1 serves about a lane a clock, so a
+ * lane without a hit asks for nothing (mixture 1,048,576, with FP32 force sums:
  * 3.0e9 accesses, 1.2 a clock, 4360 us; without them 2.3e9, 4180), and the
  * table headers lie in LDS (1.6e9, 3670), copied once per PT_WAVES waves.
  * The filter costs 5/256 VALU instructions per candidate, against 27/64 at
  * 45 % lane use for the walk along the sorted windows that it replaced.
- * Kernel time with that walk and now, us: mixture 1,048,576 atoms 4695, 3670;
- * 99,991 atoms 929, 440; 4,000 atoms 618, 114; argon 1,048,576 atoms 1290,
- * 720; 32,000 atoms 190, 53; 4,000 atoms 82, 28; water 64,000 atoms 555, 327.
+ * Time with that walk and now (HIP events around the kernel and the fold of
+ * split owners, perturbed lattices), us: mixture 1,048,576 atoms 4695, 3830;
+ * 99,991 atoms 929, 445; 4,000 atoms 618, 116; argon 1,048,576 atoms 1290,
+ * 770; 32,000 atoms 190, 56; 4,000 atoms 82, 34; water 64,000 atoms 555, 337.
  * Also measured, mixture 1,048,576, before the headers lay in LDS: both sides
  * dealt evenly (3350 us, but the energies' FP32 sums then run in another
  * order, up to 2e-6 of the total off where it cancels); the j hits levelling
